@@ -70,6 +70,11 @@ struct GemvArgs {
   // group] (np_out >= the number of column groups)
   float *pmax_out;
   int np_out;
+  // 16-bit matrix-core GEMM: when set, the fp32 rows behind the 16-bit parts
+  // (stride ldaf); an output that the parts make NaN is then summed again from
+  // them, so that weights that are not finite give what an fp32 sum gives
+  const float *Af;
+  int ldaf;
 };
 
 // Weight types
@@ -91,6 +96,9 @@ hipError_t gemv_generic(const GemvArgs &a, int wt, int epi, hipStream_t s);
 // (K % 16, lda % 16, 16-byte aligned A / W / W2).
 constexpr int kGemmMinM = 16;
 bool gemm_i8_ok(const GemvArgs &a, int epi);
+// any K from 16 and any alignment (unaligned 16-byte loads): what the
+// launchers below take; gemm_i8_ok shapes run faster
+bool gemm_i8_any_ok(const GemvArgs &a, int epi);
 hipError_t gemm_i8(const GemvArgs &a, int epi, hipStream_t s);
 // the same with the row tile forced: bm 32, 64 or 128 (0: gemm_i8's choice)
 hipError_t gemm_i8_tile(const GemvArgs &a, int epi, int bm, hipStream_t s);
@@ -115,6 +123,7 @@ hipError_t gemm_i8_skinny_q(const GemvArgs &a, int epi, hipStream_t s);
 // W / W2.
 int w16_parts(int wt);
 bool gemm_w16_ok(const GemvArgs &a, int wt, int epi);
+bool gemm_w16_any_ok(const GemvArgs &a, int wt, int epi);  // any K from 8, any alignment
 hipError_t gemm_w16(const GemvArgs &a, int wt, int epi, uint16_t *parts, int ldp, float *rs, hipStream_t s);
 hipError_t gemm_w16_tile(const GemvArgs &a, int wt, int epi, int bm, uint16_t *parts, int ldp, float *rs,
                          hipStream_t s);

@@ -34,6 +34,11 @@
 // bytes apart, so the 16-byte fragment reads of 8 consecutive lanes (16 rows,
 // same k) fall on distinct banks.  The activation tile holds NP parts (1 for
 // int8, 2 for fp16, 3 for bf16), part-major.
+// Rows whose length is no multiple of 16 bytes (and operands at any address)
+// take the register-staged form with unaligned 16-byte loads, the chunk that a
+// row ends in loaded from the row's last 16 bytes and its other bytes zeroed:
+// 333 x 1000 x 777 int8 took 970 us in the one-thread-per-output kernel that
+// these shapes had, its byte loads serial.
 //
 // MFMA lane layout (16x16x64 i8 and 16x16x32 f16 / bf16, checked on the
 // device): lane l supplies row l % 16 of A (column l % 16 of B) with the 16
@@ -41,6 +46,8 @@
 // D[4*(l/16) + r][l % 16] in accumulator register r.
 #include "ec_device.h"
 #include "ec_kernels.h"
+
+#include <float.h>
 
 namespace ec {
 
@@ -84,6 +91,41 @@ struct MfmaOp<OP_BF16> {
                                                    0);
   }
 };
+
+// 16 bytes at any address (gfx950 loads them unaligned in one instruction):
+// rows whose length is no multiple of 16 bytes start anywhere
+typedef v4i v4i_u __attribute__((aligned(1)));
+__device__ __forceinline__ v4i ld16(const int8_t *p) { return *reinterpret_cast<const v4i_u *>(p); }
+
+// The chunk [c, c + 16) of a row of KB bytes, as loaded from min(c, KB - 16):
+// the bytes that belong to it, the others zeroed.  Past the row (c >= KB) that
+// is nothing; a chunk that the row ends in was loaded from KB - 16, so its
+// bytes are the last KB - c, and the first ones belong to the chunk before.
+// Both operands' chunks are loaded from the same place, so byte j of one still
+// meets byte j of the other.
+__device__ __forceinline__ v4i tail16(v4i v, int c, int KB) {
+  const int cut = c + 16 - KB;  // bytes to clear from the front
+#pragma unroll
+  for (int d = 0; d < 4; d++) {
+    const int n = min(max(cut - 4 * d, 0), 4);
+    v[d] = n >= 4 ? 0 : (int)((uint32_t)v[d] & (0xFFFFFFFFu << (8 * n)));
+  }
+  return v;
+}
+
+// The fp32 dot of activation row m with weight row n in order, for an output
+// whose 16-bit parts gave NaN: a weight that is not finite times a part that is
+// zero, or infinities of both signs among the parts.  Only where the caller
+// gives the fp32 rows (a.Af).
+template <int OP>
+__device__ __forceinline__ float redo_dot(const GemvArgs &a, const void *W, int m, int n) {
+  const float *x = a.Af + (size_t)m * a.ldaf;
+  const uint16_t *w = reinterpret_cast<const uint16_t *>(W) + (size_t)n * a.K;
+  float s = 0.0f;
+#pragma unroll 1
+  for (int k = 0; k < a.K; k++) s = __builtin_fmaf(x[k], w2f<OP == OP_BF16>(w[k]), s);
+  return s;
+}
 
 // NB stage buffers (2, or up to 4 in the direct-to-LDS form); the
 // direct-to-LDS form (DL) has unpadded rows
@@ -156,7 +198,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   float e_as[TI][4], e_bs[JO], e_bv[JO], e_bs2[JO];
   float e_old[RES ? TI : 1][RES ? JO : 1][4];
   {
-    const float *stand = (const float *)a.W;  // N*K >= 4N bytes: valid for every column index
+    // N*K >= 4N bytes: valid for every column index (weights at odd addresses: the output's row 0)
+    const float *stand = ((uintptr_t)a.W & 3) ? a.out : (const float *)a.W;
     const float *wsp = a.ws ? a.ws : stand, *bvp = a.bias ? a.bias : stand;
     const float *ws2p = (SWI && a.ws2) ? a.ws2 : stand;
 #pragma unroll
@@ -219,13 +262,20 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     kl = k0;
 #pragma unroll
     for (int j = 0; j < ACH; j++)
-      ra[j] = *reinterpret_cast<const v4i *>(arow[j] + min(k0 + 16 * acol[j], KB - 16));
+      ra[j] = ld16(arow[j] + min(k0 + 16 * acol[j], KB - 16));
 #pragma unroll
     for (int j = 0; j < BCH; j++)
-      rb[j] = *reinterpret_cast<const v4i *>(brow[j] + min(k0 + 16 * bcol[j], KB - 16));
+      rb[j] = ld16(brow[j] + min(k0 + 16 * bcol[j], KB - 16));
   };
+  const bool rag = KB & 15;  // the row ends inside a chunk
   auto store = [&](int buf) {
     const v4i z = {0, 0, 0, 0};
+    if (rag) {
+#pragma unroll
+      for (int j = 0; j < ACH; j++) ra[j] = tail16(ra[j], kl + 16 * acol[j], KB);
+#pragma unroll
+      for (int j = 0; j < BCH; j++) rb[j] = tail16(rb[j], kl + 16 * bcol[j], KB);
+    }
 #pragma unroll
     for (int j = 0; j < ACH; j++)
       *reinterpret_cast<v4i *>(la + buf * NP * BM * kPitch + aoff[j]) = kl + 16 * acol[j] < KB ? ra[j] : z;
@@ -432,6 +482,37 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     if (t == 0) __hip_atomic_store(&gm_cnt[tl], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
+  if constexpr (!I8) {
+    if (a.Af) {  // uniform
+      bool bad = false;
+#pragma unroll
+      for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) {
+          const v4f w = acc[i][j];
+          bad = bad || w[0] != w[0] || w[1] != w[1] || w[2] != w[2] || w[3] != w[3];
+        }
+      if (bad) {  // this thread's outputs one by one
+#pragma unroll 1
+        for (int q = 0; q < TI * JO * 4; q++) {
+          const int m = lrow0 + 16 * (q / (4 * JO)) + (q & 3), n = lcol0 + 16 * ((q >> 2) % JO);
+          if (m >= M || n >= N) continue;
+          float x = redo_dot<OP>(a, a.W, m, n);
+          float *o = a.out + (size_t)m * a.ldo + n;
+          if constexpr (SWI) {
+            x = silu(x, etab) * redo_dot<OP>(a, a.W2, m, n);
+          } else {
+            if (a.bias) x = x + a.bias[n];
+            if constexpr (RES) x = *o + x;
+            if constexpr (GELU) x = gelu_new(x);
+          }
+          *o = x;
+        }
+        return;
+      }
+    }
+  }
+
   // ---- epilogue: lane holds D[4*lq + r][lr] of each tile ----
   // Every value of a column tile is computed before any of its stores, so
   // that the 4*TI independent chains (SiLU's expf and division, GELU's tanh)
@@ -492,6 +573,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   }
 }
 
+bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
+
 #ifndef EC_GEMM_DL
 #define EC_GEMM_DL 1
 #endif
@@ -518,7 +601,8 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   // split K for few tiles over long rows: C2's 128-token down projection
   // (24 tiles of 32 x 128 over 48 stages of K) ran each tile's whole K on
   // one CU while 232 CUs idled
-  const bool dl = EC_GEMM_DL && (a.K * MfmaOp<OP>::EB) % kBK == 0 && (a.lda * MfmaOp<OP>::EB) % kBK == 0;
+  const bool dl = EC_GEMM_DL && (a.K * MfmaOp<OP>::EB) % kBK == 0 && (a.lda * MfmaOp<OP>::EB) % kBK == 0 &&
+                  aligned16(a.A) && aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2));
   const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM) : 1;
   const dim3 grid(8 * ((T + 7) / 8), ks);
   if constexpr (BM == 32) {
@@ -580,12 +664,14 @@ bool epi_ok(int epi) {
          epi == EPI_BIAS_RESID || epi == EPI_BIAS_GELU;
 }
 
-bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
-
-// bf16 bits of x rounded to nearest even (finite x)
-__device__ __forceinline__ uint16_t f2b_rne(float x) {
+// bf16 bits of x rounded to nearest even; the largest finite values, which
+// would round to infinity, are cut instead (the next part takes what is left),
+// infinities stay and NaN becomes the quiet one
+__device__ __forceinline__ uint16_t f2b_part(float x) {
   const uint32_t u = __builtin_bit_cast(uint32_t, x);
-  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+  const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+  if (x != x) return 0x7fc0;
+  return (uint16_t)((r & 0x7fffu) == 0x7f80u ? u >> 16 : r);
 }
 
 // one block of 256 threads per row: the row's 16-bit parts and scale
@@ -597,31 +683,35 @@ __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int
   const float *row = x + (size_t)m * ldx;
   if constexpr (OP == OP_F16) {
     float mx = 0.0f;
-    for (int k = t; k < K; k += 256) mx = fmaxf(mx, fabsf(row[k]));
+    for (int k = t; k < K; k += 256) {
+      const float v = fabsf(row[k]);
+      mx = fmaxf(mx, v <= FLT_MAX ? v : 0.0f);
+    }
     mx = block_max256(mx, red);
-    // 2^-e x in [2^14, 2^15) for the row's largest |x|; zero, tiny and
-    // non-finite rows keep e = 0 (values pass through the fp16 parts)
+    // 2^-e x in [2^14, 2^15) for the row's largest finite |x|; zero rows keep
+    // e = 0, tiny ones e = -100.  A value that is not finite is its first
+    // part, the others zero.
     int e = 0;
-    if (mx > 0.0f && mx <= 3.402823466e38f) e = max(ilogbf(mx) - 14, -100);
+    if (mx > 0.0f) e = max(ilogbf(mx) - 14, -100);
     uint16_t *h = out + (size_t)m * 2 * ldo, *l = h + ldo;
     for (int k = t; k < K; k += 256) {
       const float v = ldexpf(row[k], -e);
       const _Float16 hi = (_Float16)v;
       h[k] = __builtin_bit_cast(uint16_t, hi);
-      l[k] = f2h(v - (float)hi);
+      l[k] = fabsf(v) <= FLT_MAX ? f2h(v - (float)hi) : (uint16_t)0;
     }
     if (t == 0) rs[m] = ldexpf(1.0f, e);
   } else {
     uint16_t *h = out + (size_t)m * 3 * ldo, *mid = h + ldo, *l = mid + ldo;
     for (int k = t; k < K; k += 256) {
       const float v = row[k];
-      const uint16_t b0 = f2b_rne(v);
-      const float r1 = v - b2f(b0);
-      const uint16_t b1 = f2b_rne(r1);
+      const uint16_t b0 = f2b_part(v);
+      const float r1 = fabsf(v) <= FLT_MAX ? v - b2f(b0) : 0.0f;
+      const uint16_t b1 = f2b_part(r1);
       const float r2 = r1 - b2f(b1);
       h[k] = b0;
       mid[k] = b1;
-      l[k] = f2b_rne(r2);
+      l[k] = f2b_part(r2);
     }
     if (t == 0) rs[m] = 1.0f;
   }
@@ -667,7 +757,9 @@ __device__ unsigned sk_cnt[kSkMaxGroups];
 // with the row scale quant_scale(max |a|) of the row maximum given as partial
 // maxima (a.pmax, a.np); the codes are quant_rows' (the same scale and the
 // same per-element code), so the floats equal the unfused GEMM's.
-template <int OP, int TI, int NJ, int EPI, bool QA = false>
+// RAG: rows may end inside a 16-byte chunk (a kernel of its own: the chunk's
+// mask spilled registers of the others)
+template <int OP, int TI, int NJ, int EPI, bool QA = false, bool RAG = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
   using Op = MfmaOp<OP>;
   using Acc = typename Op::Acc;
@@ -680,7 +772,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
   static_assert(!QA || I8, "fused quantization of int8 activations");
   constexpr int NB = SWI ? 2 : NJ;  // B tiles: NJ tiles of 16 rows, or 16 gate + 16 up rows
   constexpr int FR = TI * NP * (QA ? 4 : 1) + NB;  // 16-byte loads per lane and step
-  constexpr int U = FR <= 3 ? 8 : FR <= 5 ? 4 : 2;  // K steps per wave in flight (within 128 VGPRs)
+  constexpr int U = (FR <= 3 ? 8 : FR <= 5 ? 4 : 2) / (RAG && FR <= 5 ? 2 : 1);  // K steps per wave in flight (within 128 VGPRs)
   __shared__ Acc part[16][TI][NB][64];  // [wave][i][j][lane]
   __shared__ uint64_t etab[SWI ? 32 : 1];
   __shared__ float s_sc[QA ? 32 : 1];  // QA: the rows' scales
@@ -775,11 +867,11 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
             for (int c = 0; c < 4; c++) ff[u][i][c] = *reinterpret_cast<const float4 *>(arowf[i] + kc + 4 * c);
           } else {
 #pragma unroll
-            for (int p = 0; p < NP; p++) fa[u][i][p] = *reinterpret_cast<const v4i *>(arow[i][p] + kc);
+            for (int p = 0; p < NP; p++) fa[u][i][p] = ld16(arow[i][p] + kc);
           }
         }
 #pragma unroll
-        for (int j = 0; j < NB; j++) fb[u][j] = *reinterpret_cast<const v4i *>(brow[j] + kc);
+        for (int j = 0; j < NB; j++) fb[u][j] = ld16(brow[j] + kc);
       }
     }
 #pragma unroll
@@ -787,6 +879,16 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
       const int st = sb + nw * u;
       if (st < ks1) {
         const bool in = 64 * st + 16 * lq < KB;
+        if (RAG && 64 * st + 64 > KB) {  // uniform: the row ends inside this step
+#pragma unroll
+          for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int p = 0; p < NP; p++) fa[u][i][p] = tail16(fa[u][i][p], 64 * st + 16 * lq, KB);
+          if constexpr (!I8) {  // a weight that is not finite would make NaN of a zero activation
+#pragma unroll
+            for (int j = 0; j < NB; j++) fb[u][j] = tail16(fb[u][j], 64 * st + 16 * lq, KB);
+          }
+        }
         if constexpr (QA) {
           // the codes of the fragment's 16 elements, packed four per word
 #pragma unroll
@@ -919,8 +1021,10 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
     }
   } else {
     v = sum[0] * as;
+    if (a.Af && v != v) v = redo_dot<OP>(a, a.W, m, n);
     if constexpr (SWI) {
-      const float u = sum[1] * as;
+      float u = sum[1] * as;
+      if (a.Af && u != u) u = redo_dot<OP>(a, a.W2, m, n);
       v = silu(v, etab) * u;
     } else if (a.bias) {
       v = v + a.bias[n];
@@ -955,7 +1059,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
   }
 }
 
-template <int OP, int TI, int NJ, int EPI, bool QA = false>
+template <int OP, int TI, int NJ, int EPI, bool QA = false, bool RAG = false>
 hipError_t launch_skinny_nj(const GemvArgs &a, int wpb, int ksplit, hipStream_t s) {
   const int ksteps = (a.K * MfmaOp<OP>::EB + 63) / 64;
   constexpr int NO = EPI == EPI_SWIGLU ? 1 : NJ;
@@ -975,7 +1079,7 @@ hipError_t launch_skinny_nj(const GemvArgs &a, int wpb, int ksplit, hipStream_t 
   if (wpb <= 0) wpb = min(16, max(4, kper / (EPI == EPI_SWIGLU ? 6 : 2)));
   wpb = max(min(wpb, 16), 4 * TI * NO);
   if (a.pmax_out && groups > a.np_out) return hipErrorInvalidValue;
-  klaunch((gemm_skinny_kernel<OP, TI, NJ, EPI, QA>), dim3(groups, ksplit), dim3(64 * wpb), 0, s, a);
+  klaunch((gemm_skinny_kernel<OP, TI, NJ, EPI, QA, RAG>), dim3(groups, ksplit), dim3(64 * wpb), 0, s, a);
   return hipGetLastError();
 }
 
@@ -988,6 +1092,8 @@ hipError_t launch_skinny_nj(const GemvArgs &a, int wpb, int ksplit, hipStream_t 
 // 7.2-7.7 us measured); down (K = 8960) goes from 12.6 to 10.2 us.
 template <int OP, int TI, int EPI, bool QA = false>
 hipError_t launch_skinny(const GemvArgs &a, int wpb, hipStream_t s) {
+  if constexpr (!QA)
+    if (a.K * MfmaOp<OP>::EB % 16) return launch_skinny_nj<OP, TI, 1, EPI, false, true>(a, wpb, 1, s);
   if constexpr (EPI != EPI_SWIGLU && TI == 1) {
     if (a.N >= 16 * 1024) return launch_skinny_nj<OP, TI, 4, EPI, QA>(a, wpb, 1, s);
     if (OP == OP_I8 && (a.N + 15) / 16 < 192 && (a.K + 63) / 64 >= 64) {
@@ -1020,6 +1126,11 @@ hipError_t launch_skinny_op(const GemvArgs &a, int epi, int wpb, hipStream_t s) 
 
 }  // namespace
 
+bool gemm_i8_any_ok(const GemvArgs &a, int epi) {
+  return a.M >= 1 && a.N >= 1 && a.K >= 16 && a.lda >= a.K && a.A && a.as && a.W && !a.cand &&
+         (epi != EPI_SWIGLU || a.W2) && epi_ok(epi);
+}
+
 bool gemm_i8_ok(const GemvArgs &a, int epi) {
   if (a.M < 1 || a.N < 1 || a.K < 16 || a.K % 16 || a.lda % 16 || !a.as || a.cand) return false;
   if (!aligned16(a.A) || !aligned16(a.W)) return false;
@@ -1028,13 +1139,18 @@ bool gemm_i8_ok(const GemvArgs &a, int epi) {
 }
 
 hipError_t gemm_i8_tile(const GemvArgs &a, int epi, int bm, hipStream_t s) {
-  if (!gemm_i8_ok(a, epi) || (bm != 0 && bm != 32 && bm != 64 && bm != 128)) return hipErrorInvalidValue;
+  if (!gemm_i8_any_ok(a, epi) || (bm != 0 && bm != 32 && bm != 64 && bm != 128)) return hipErrorInvalidValue;
   return launch_op<OP_I8>(a, epi, bm, s);
 }
 
 hipError_t gemm_i8(const GemvArgs &a, int epi, hipStream_t s) { return gemm_i8_tile(a, epi, 0, s); }
 
 int w16_parts(int wt) { return wt == WT_BF16 ? 3 : 2; }
+
+bool gemm_w16_any_ok(const GemvArgs &a, int wt, int epi) {
+  return (wt == WT_F16 || wt == WT_BF16) && a.M >= 1 && a.N >= 1 && a.K >= 8 && a.lda >= a.K && a.A && a.W &&
+         !a.cand && !a.ws && !a.ws2 && (epi != EPI_SWIGLU || a.W2) && epi_ok(epi);
+}
 
 bool gemm_w16_ok(const GemvArgs &a, int wt, int epi) {
   if (wt != WT_F16 && wt != WT_BF16) return false;
@@ -1055,7 +1171,7 @@ hipError_t split_rows16(const GemvArgs &a, int wt, uint16_t *parts, int ldp, flo
 
 hipError_t gemm_w16_parts(const GemvArgs &a, int wt, int epi, int bm, const uint16_t *parts, int ldp,
                           const float *rs, hipStream_t s) {
-  if (!gemm_w16_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
+  if (!gemm_w16_any_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
     return hipErrorInvalidValue;
   if (!parts || !rs || ldp < a.K || ldp % 8 || !aligned16(parts)) return hipErrorInvalidValue;
   GemvArgs q = a;
@@ -1078,7 +1194,7 @@ hipError_t gemm_w16_parts(const GemvArgs &a, int wt, int epi, int bm, const uint
 
 hipError_t gemm_w16_tile(const GemvArgs &a, int wt, int epi, int bm, uint16_t *parts, int ldp, float *rs,
                          hipStream_t s) {
-  if (!gemm_w16_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
+  if (!gemm_w16_any_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
     return hipErrorInvalidValue;
   hipError_t e = split_rows16(a, wt, parts, ldp, rs, s);
   if (e != hipSuccess) return e;
@@ -1091,7 +1207,7 @@ hipError_t gemm_w16(const GemvArgs &a, int wt, int epi, uint16_t *parts, int ldp
 
 
 hipError_t gemm_i8_skinny(const GemvArgs &a, int epi, int wpb, hipStream_t s) {
-  if (!gemm_i8_ok(a, epi) || a.M > 32 || wpb < 0 || wpb > 16) return hipErrorInvalidValue;
+  if (!gemm_i8_any_ok(a, epi) || a.M > 32 || wpb < 0 || wpb > 16) return hipErrorInvalidValue;
   return launch_skinny_op<OP_I8>(a, epi, wpb, s);
 }
 

@@ -1,0 +1,107 @@
+"""GEMMs whose rows are no whole number of 16-byte chunks, or whose operands lie
+at any address: the matrix-core kernels' unaligned loads and the mask of the
+chunk that a row ends in, against the oracle (int8: bit for bit; 16-bit: the
+fp32 bound of tests/test_gpu_kernels.py), and, for values that are not finite,
+the class (finite, which infinity, NaN) of an fp32 sum."""
+import numpy as np
+import pytest
+
+import edgecore_amd as ec
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+# rows: one, both skinny fragments and their edges, the tiles' edges; widths:
+# one byte (element) past and short of a chunk, a 64-byte step, a 128-byte stage
+SHAPES = [(1, 17, 33), (1, 1001, 777), (15, 31, 16), (16, 65, 100), (17, 1000, 129), (32, 127, 15), (33, 129, 40),
+          (64, 1000, 130), (65, 255, 257), (300, 1023, 700), (130, 4097, 65), (600, 1001, 9001)]
+
+
+def _dev(fn, out_shape, *args):
+    out = ec.DeviceBuffer(4 * int(np.prod(out_shape)))
+    try:
+        assert fn(out.ptr, *args) == 0, ec.last_error()
+        assert ec.lib().ec_sync() == 0
+        return out.to_array(np.float32, out_shape)
+    finally:
+        out.close()
+
+
+def _at(a, off):
+    """A device copy of `a` that starts `off` bytes into its allocation."""
+    raw = np.concatenate([np.zeros(off, np.uint8), np.ascontiguousarray(a).view(np.uint8).reshape(-1)])
+    return ec.DeviceBuffer.from_array(raw)
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+def test_int8_bit_exact(M, K, N):
+    rng = np.random.default_rng(M + 3 * K + N)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    a_s, b_s = rng.uniform(1e-4, 1e-1, M).astype(np.float32), rng.uniform(1e-4, 1e-2, N).astype(np.float32)
+    bias = rng.normal(0, 0.02, N).astype(np.float32) if M % 2 else None
+    got = ec.gemm_int8(A, a_s, B, b_s, bias)
+    assert np.array_equal(got.view(np.uint32), oracle.gemm_int8(A, a_s, B, b_s, bias).view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 96, 40), (20, 128, 130), (40, 128, 130), (40, 100, 33)])
+@pytest.mark.parametrize("oa,ob", [(1, 0), (0, 3), (8, 4)])
+def test_int8_any_address(M, K, N, oa, ob):
+    rng = np.random.default_rng(M + K + N + oa)
+    A = rng.integers(-128, 128, (M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    a_s = rng.uniform(1e-4, 1e-1, M).astype(np.float32)
+    bufs = [_at(A, oa), ec.DeviceBuffer.from_array(a_s), _at(B, ob)]
+    try:
+        got = _dev(ec.lib().ec_gemm_int8_dev, (M, N), bufs[0].ptr + oa, bufs[1].ptr, bufs[2].ptr + ob, None, None, M,
+                   K, N)
+    finally:
+        for b in bufs:
+            b.close()
+    assert np.array_equal(got.view(np.uint32), oracle.gemm_int8(A, a_s, B, None, None).view(np.uint32))
+
+
+def _bits(x, bf16):
+    if not bf16:
+        return np.asarray(x, np.float16).view(np.uint16)
+    u = np.asarray(x, np.float32).view(np.uint32).astype(np.uint64)
+    return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES[:-1])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_w16_within_bound(M, K, N, bf16):
+    rng = np.random.default_rng(M + K + N + bf16)
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    B = _bits(rng.normal(0, 0.02, (N, K)), bf16)
+    got = (ec.gemm_bf16_fp32 if bf16 else ec.gemm_fp16_fp32)(A, B)
+    Bf = (B.astype(np.uint32) << 16).view(np.float32) if bf16 else B.view(np.float16).astype(np.float32)
+    want = A.astype(np.float64) @ Bf.astype(np.float64).T
+    bound = 2.0 * K * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(Bf).astype(np.float64).T)
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("M", [5, 40])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_w16_not_finite(M, bf16):
+    """Infinities and NaN in single activations and weights: every output is
+    of the class that the fp32 sum over its row gives (finite ones within the
+    bound)."""
+    K, N = 101, 50
+    rng = np.random.default_rng(M + bf16)
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    W = rng.normal(0, 0.02, (N, K)).astype(np.float32)
+    A[0, 3], A[1, K - 1], A[2, 50] = np.inf, -np.inf, np.nan
+    W[0, 100], W[7, 3], W[9, 20] = np.inf, -np.inf, np.nan
+    W[11, 3] = 0.0  # meets the infinity of row 0
+    B = _bits(W, bf16)
+    Bf = (B.astype(np.uint32) << 16).view(np.float32) if bf16 else B.view(np.float16).astype(np.float32)
+    got = (ec.gemm_bf16_fp32 if bf16 else ec.gemm_fp16_fp32)(A, B)
+    with np.errstate(invalid="ignore"):
+        want = (A[:, None, :].astype(np.float64) * Bf[None].astype(np.float64)).sum(2)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert inf.any() and np.array_equal(got[inf], want[inf].astype(np.float32))
+    mag = np.where(np.isfinite(A), np.abs(A), 0).astype(np.float64) @ np.where(np.isfinite(Bf), np.abs(Bf), 0).T
+    assert np.all(np.abs(got[fin] - want[fin]) <= 2.0 * K * 2.0 ** -24 * mag[fin])
