@@ -107,3 +107,40 @@ def test_driver_sampling_equals_full_row_replay(make_model, tmp_path):
             ids.append(cur)
             pos += 1
     assert got == ids
+
+
+@pytest.mark.parametrize("V", [131, 4095, 4096, 8193, 50257])
+@pytest.mark.parametrize("top_k", [1, 31, 128])
+def test_topk_selection_edges(V, top_k):
+    """The threshold's list at its edges: about as many equal largest values as
+    the list holds (512) and more, which the block sorts; the largest values
+    all in one thread's share (columns 512 or 1024 apart); rows in descending
+    and ascending order; nothing but -inf and the lowest finite value."""
+    rng = np.random.default_rng(V * 3 + top_k)
+    base = rng.normal(0, 1, V).astype(np.float32)
+    rows = [np.sort(base), np.sort(base)[::-1].copy()]
+    for m in (511, 512, 513, 600, 2000):
+        r = base.copy()
+        r[rng.permutation(V)[:min(m, V)]] = 9.0
+        rows.append(r)
+    for step in (512, 1024):
+        r = base.copy()
+        r[3::step] += 50.0
+        rows.append(r)
+    r = np.full(V, -np.inf, np.float32)
+    r[::7] = np.finfo(np.float32).min
+    rows.append(r)
+    L = np.stack(rows)
+    vals, idx, status = ec.topk_dev(L, top_k)
+    buf = ec.DeviceBuffer.from_array(L)
+    v2, i2, s2 = np.empty_like(vals), np.empty_like(idx), np.empty_like(status)
+    try:
+        assert ec.lib().ec_topk_dev_noalloc(buf.ptr, len(rows), V, V, top_k, v2.ctypes.data, i2.ctypes.data,
+                                            s2.ctypes.data) == 0, ec.last_error()
+    finally:
+        buf.close()
+    assert np.array_equal(vals, v2) and np.array_equal(idx, i2) and np.array_equal(status, s2)
+    for i, row in enumerate(rows):
+        wv, wi = _np_topk(row, top_k + 1)
+        assert status[i] == _status(row, top_k), i
+        assert np.array_equal(vals[i], wv) and np.array_equal(idx[i], wi), i
