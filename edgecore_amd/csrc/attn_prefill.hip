@@ -14,26 +14,27 @@
 // reference's order differs from it by the last bits of a double, below what
 // the float rounding of pr_p resolves except in rare ties.
 //
-// One block takes one query head and NW * QW consecutive tokens: NW waves of
-// QW tokens each (8 x 2 when the scores fit the LDS, else 8 x 1 or 4 x 1).
-// The keys of all of them are staged through LDS 64 positions at a time,
-// converted to fp32 once for the block:
-//   - scores: lane = position; each lane runs its position's sequential dots
-//     for the wave's QW tokens off one read of the K row (q in registers); K
-//     rows are head_dim + 4 floats apart, so the 16-byte reads of 8 lanes hit
-//     distinct banks;
+// Two kernels: attn_prefill_mm_kernel (below), with the products on the matrix
+// cores, for spans of up to 4096 positions, and attn_prefill_kernel for longer
+// ones and for short prompts at head_dim 128.
+//
+// attn_prefill_kernel: one block takes one query head and NW consecutive
+// tokens, one per wave (8, or 4 when the scores of 8 do not fit the LDS).  The
+// keys of all of them are staged through LDS 64 positions at a time, converted
+// to fp32 once for the block:
+//   - scores: lane = position; each lane runs its position's sequential dot
+//     off its K row (q in registers); K rows are head_dim + 4 floats apart, so
+//     the 16-byte reads of 8 lanes hit distinct banks;
 //   - softmax: per token, inside its wave, four of a lane's positions per
 //     step (expf without branches);
-//   - output: lane = element d; the wave adds pr_p * v_p[d] for its QW tokens
-//     in position order from V tiles staged transposed (a lane's positions
-//     contiguous, 16-byte reads of four).  A tile that every token of a
-//     two-token wave takes whole runs as one asm block whose probabilities
-//     come from one read per token and a DPP row broadcast per product;
-//     partial tiles read the probabilities by quad, the next quad's reads in
+//   - output: lane = element d; the wave adds pr_p * v_p[d] in position order
+//     from V tiles staged transposed (a lane's positions contiguous, 16-byte
+//     reads of four), the probabilities read by quad, the next quad's reads in
 //     flight during the current quad's adds.
 // The blocks with the longest key ranges start first; the grid is (head,
 // token group), which spreads the blocks over all 8 XCDs.
 #include <cfloat>
+#include <type_traits>
 
 #include "ec_device.h"
 #include "ec_expf.h"
@@ -44,379 +45,6 @@ namespace ec {
 namespace {
 
 constexpr int kPfTile = 64;  // positions per staged K / V tile
-
-// The output sums of two tokens over 8*n8 positions (n8 >= 1), in order:
-// o_i += pr_i[p] * v[p] (product rounded, then the add) for token i = 0, 1.
-// p0/p1: LDS byte addresses of the tokens' probabilities of the first
-// position, va: of this lane's element of that position in the transposed V
-// tile (all 16-byte aligned).  The reads of the next four positions are in
-// flight while the current four are added.  Reads four positions past the end
-// (values unused).
-__device__ __forceinline__ void pf_chain2(float &o0, float &o1, uint32_t p0, uint32_t p1, uint32_t va, int n8) {
-  float t0, t1;
-  asm volatile(
-      "ds_read_b128 v[40:43], %[p0] offset:0\n"
-      "ds_read_b128 v[44:47], %[p1] offset:0\n"
-      "ds_read_b128 v[48:51], %[va] offset:0\n"
-      "L_pf_chain%=:\n"
-      "ds_read_b128 v[52:55], %[p0] offset:16\n"
-      "ds_read_b128 v[56:59], %[p1] offset:16\n"
-      "ds_read_b128 v[60:63], %[va] offset:16\n"
-      "s_waitcnt lgkmcnt(3)\n"
-      "v_mul_f32 %[t0], v40, v48\n"
-      "v_mul_f32 %[t1], v44, v48\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v41, v49\n"
-      "v_mul_f32 %[t1], v45, v49\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v42, v50\n"
-      "v_mul_f32 %[t1], v46, v50\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v43, v51\n"
-      "v_mul_f32 %[t1], v47, v51\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_add_u32 %[p0], 32, %[p0]\n"
-      "v_add_u32 %[p1], 32, %[p1]\n"
-      "v_add_u32 %[va], 32, %[va]\n"
-      "ds_read_b128 v[40:43], %[p0] offset:0\n"
-      "ds_read_b128 v[44:47], %[p1] offset:0\n"
-      "ds_read_b128 v[48:51], %[va] offset:0\n"
-      "s_waitcnt lgkmcnt(3)\n"
-      "v_mul_f32 %[t0], v52, v60\n"
-      "v_mul_f32 %[t1], v56, v60\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v53, v61\n"
-      "v_mul_f32 %[t1], v57, v61\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v54, v62\n"
-      "v_mul_f32 %[t1], v58, v62\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32 %[t0], v55, v63\n"
-      "v_mul_f32 %[t1], v59, v63\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_sub_u32 %[n], %[n], 1\n"
-      "s_cmp_lg_u32 %[n], 0\n"
-      "s_cbranch_scc1 L_pf_chain%=\n"
-      "s_waitcnt lgkmcnt(0)\n"
-      : [o0] "+v"(o0), [o1] "+v"(o1), [t0] "=&v"(t0), [t1] "=&v"(t1), [p0] "+v"(p0), [p1] "+v"(p1), [va] "+v"(va),
-        [n] "+s"(n8)
-      :
-      : "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "scc", "memory");
-}
-
-// The output sums of two tokens over one whole tile of 64 positions, in
-// order, as pf_chain2.  p0/p1: LDS byte addresses of the tokens'
-// probabilities of positions 4*(lane % 16) .. +3 of the tile, so that lane j
-// of every 16-lane row holds those of quad j; each product takes its
-// probability from that lane by a DPP row broadcast (row_newbcast), which
-// replaces a 64-lane broadcast read per quad and token.  va: LDS byte address
-// of this lane's element of the tile's first position in the transposed V
-// tile; quad j is read 16*j bytes further, eight quads ahead of its adds.
-__device__ __forceinline__ void pf_tile2(float &o0, float &o1, uint32_t p0, uint32_t p1, uint32_t va) {
-  float t0, t1;
-  asm volatile(
-      "ds_read_b128 v[40:43], %[p0]\n"
-      "ds_read_b128 v[44:47], %[p1]\n"
-      "ds_read_b128 v[48:51], %[va] offset:0\n"
-      "ds_read_b128 v[52:55], %[va] offset:16\n"
-      "ds_read_b128 v[56:59], %[va] offset:32\n"
-      "ds_read_b128 v[60:63], %[va] offset:48\n"
-      "ds_read_b128 v[64:67], %[va] offset:64\n"
-      "ds_read_b128 v[68:71], %[va] offset:80\n"
-      "ds_read_b128 v[72:75], %[va] offset:96\n"
-      "ds_read_b128 v[76:79], %[va] offset:112\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v48 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v48 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v49 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v49 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v50 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v50 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v51 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v51 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[48:51], %[va] offset:128\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v52 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v52 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v53 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v53 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v54 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v54 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v55 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v55 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[52:55], %[va] offset:144\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v56 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v56 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v57 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v57 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v58 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v58 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v59 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v59 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[56:59], %[va] offset:160\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v60 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v60 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v61 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v61 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v62 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v62 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v63 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v63 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[60:63], %[va] offset:176\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v64 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v64 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v65 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v65 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v66 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v66 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v67 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v67 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[64:67], %[va] offset:192\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v68 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v68 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v69 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v69 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v70 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v70 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v71 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v71 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[68:71], %[va] offset:208\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v72 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v72 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v73 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v73 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v74 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v74 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v75 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v75 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[72:75], %[va] offset:224\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v76 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v76 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v77 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v77 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v78 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v78 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v79 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v79 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "ds_read_b128 v[76:79], %[va] offset:240\n"
-      "s_waitcnt lgkmcnt(7)\n"
-      "v_mul_f32_dpp %[t0], v40, v48 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v48 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v49 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v49 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v50 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v50 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v51 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v51 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(6)\n"
-      "v_mul_f32_dpp %[t0], v40, v52 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v52 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v53 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v53 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v54 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v54 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v55 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v55 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(5)\n"
-      "v_mul_f32_dpp %[t0], v40, v56 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v56 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v57 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v57 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v58 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v58 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v59 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v59 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(4)\n"
-      "v_mul_f32_dpp %[t0], v40, v60 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v60 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v61 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v61 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v62 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v62 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v63 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v63 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(3)\n"
-      "v_mul_f32_dpp %[t0], v40, v64 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v64 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v65 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v65 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v66 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v66 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v67 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v67 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(2)\n"
-      "v_mul_f32_dpp %[t0], v40, v68 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v68 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v69 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v69 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v70 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v70 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v71 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v71 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(1)\n"
-      "v_mul_f32_dpp %[t0], v40, v72 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v72 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v73 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v73 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v74 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v74 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v75 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v75 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "s_waitcnt lgkmcnt(0)\n"
-      "v_mul_f32_dpp %[t0], v40, v76 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v44, v76 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v41, v77 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v45, v77 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v42, v78 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v46, v78 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      "v_mul_f32_dpp %[t0], v43, v79 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_mul_f32_dpp %[t1], v47, v79 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      "v_add_f32 %[o0], %[o0], %[t0]\n"
-      "v_add_f32 %[o1], %[o1], %[t1]\n"
-      : [o0] "+v"(o0), [o1] "+v"(o1), [t0] "=&v"(t0), [t1] "=&v"(t1)
-      : [p0] "v"(p0), [p1] "v"(p1), [va] "v"(va)
-      : "v40", "v41", "v42", "v43", "v44", "v45", "v46", "v47", "v48", "v49", "v50", "v51", "v52", "v53", "v54", "v55", "v56", "v57", "v58", "v59", "v60", "v61", "v62", "v63", "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77", "v78", "v79", "memory");
-}
 
 // V tiles are staged transposed: element d of the tile's position r at
 // tile[pf_vrow(d) + r].  Rows are 68 floats apart plus 4 more every 8 rows,
@@ -656,14 +284,6 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
     };
     const int r0 = max(p0, lo[0]), r1 = min(p0 + kPfTile - 1, pos[QW - 1]);
     int c0 = max(p0, lo[QW - 1]), c1 = min(p0 + kPfTile - 1, pos[0]);  // taken by every token
-    if constexpr (QW == 2 && DPL == 1) {
-      if (c0 == p0 && c1 == p0 + kPfTile - 1) {  // the whole tile, for both tokens
-        const int pq = p0 - lo0 + 4 * (lane & 15);
-        pf_tile2(o[0][0], o[1][0], (uint32_t)(uintptr_t)(scq[0] + pq), (uint32_t)(uintptr_t)(scq[QW - 1] + pq),
-                 (uint32_t)(uintptr_t)vt);
-        continue;
-      }
-    }
     if (c0 > c1) c0 = r1 + 1, c1 = r1;
     int p = r0;
     for (; p < c0; p++) add_some(p);
@@ -676,17 +296,6 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
       // reads are unconditional; past c1 they reach at most 4 positions
       // further: the tile's 4 spare rows, the next token's score slots or the
       // 4 spare floats after the last token's (values not used).
-      if constexpr (QW == 2 && DPL == 1) {
-        // the two-token, one-element case (the long prompts) in one asm loop
-        // of 8 positions per iteration; an odd group and the tail below
-        const int n8 = __builtin_amdgcn_readfirstlane(ng >> 1);
-        if (n8 > 0) {
-          pf_chain2(o[0][0], o[1][0], (uint32_t)(uintptr_t)(scq[0] + (p - lo0)),
-                    (uint32_t)(uintptr_t)(scq[QW - 1] + (p - lo0)), (uint32_t)(uintptr_t)(vt + (p - p0)), n8);
-          p += 8 * n8;
-        }
-        for (int e = 0; e < 4 * (ng & 1); e++, p++) add_some(p);
-      } else {
       float4 pa[QW], pb[QW];
       float va[4][DPL], vb[4][DPL];
       auto load4 = [&](int pp, float4 *pr, float (*vv)[DPL]) {
@@ -731,7 +340,6 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
         p += 4;
         if (++g == ng) break;
       }
-      }
     }
     for (; p <= r1; p++) add_some(p);
   }
@@ -743,6 +351,396 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
       for (int j = 0; j < DPL; j++) out[64 * j] = o[i][j];
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Up to 4096 positions: the products on the matrix cores.
+//
+// v_mfma_f32_16x16x1_4b_f32 with a zero addend gives, per instruction, four
+// 16 x 16 outer products whose elements are single rounded fp32 products (equal
+// to v_mul_f32 bit for bit on 5 M random bit patterns, subnormals included), so
+// such a product and a v_add_f32 keep the reference's order and rounding, and
+// the instruction broadcasts its operands itself: no LDS broadcast reads, no
+// DPP products.  What it does not do is run beside the adds (fp32 matrix
+// instructions use the vector ALUs): 34 cycles for 1024 products, then 16 adds
+// of 2.4 cycles, 4.4 cycles per product and add of 64 lanes with two or more
+// waves per SIMD, against 6.4 for a DPP product and its add.  (The f16 forms do
+// run beside the adds, but the sum of a factor's three 16-bit parts' products
+// is not the rounded product: 19% of them off by a last bit.)
+//
+// One block takes 16 consecutive tokens of one query head, 8 waves.
+//   - scores: tile t of 64 positions belongs to wave t % 8, which keeps its
+//     16 x 64 scores in 16 registers per lane (up to NT tiles): scores never
+//     reach LDS, so two blocks share a CU where 16 tokens' scores of 2048
+//     positions (128 KB) left room for one.  B = the lane's position's k row,
+//     A = four elements of the 16 tokens' q, one of them broadcast to the four
+//     blocks per product.  Register 4 b + r of lane l: token 4 (l / 16) + r,
+//     position 16 b + l % 16.
+//   - softmax on those registers; maxima and double sums over the 16 lanes of
+//     a DPP row, then over the waves.
+//   - output: wave w < head_dim / 16 owns elements 16 w .. 16 w + 15 of the 16
+//     tokens.  The probabilities of 8 tiles (written by their owners) are in
+//     LDS in operand order, 64 floats per four positions, the values come
+//     straight from the cache; the four blocks of a product are four
+//     positions, whose products are added in order to the lane's four tokens.
+// A masked product is replaced by -0 (x + -0 == x), so a value that is not
+// finite outside a token's range does not reach it.
+//
+// 2048 tokens, 14 heads of 64: 363 us with the scores in LDS and DPP products,
+// 252 us here; 12 heads of 128: 667 and 319 us; 500 tokens, 14 heads: 54 and
+// 43 us.  The adds and products alone are about 125 us of that at 2.3 GHz, the
+// exponentials 25 us; the rest is the output phase's one wave per SIMD and
+// block (198 cycles per four positions where the SIMD could do 72).
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kMmTok = 16;  // tokens per block
+
+template <int ABID>
+__device__ __forceinline__ v16f mm_bcast(float a, float b) {  // block ABID of a to all four
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, v16f{0}, 2, ABID, 0);
+}
+
+// the tile registers by a uniform index: a branch per tile (a move of 16
+// registers in the taken one)
+template <int NT>
+__device__ __forceinline__ v16f mm_get(const v16f (&S)[NT], int k) {
+  v16f v = S[0];
+#pragma unroll
+  for (int i = 1; i < NT; i++)
+    if (k == i) {
+      v = S[i];
+      asm volatile("" : "+v"(v));
+    }
+  return v;
+}
+template <int NT>
+__device__ __forceinline__ void mm_put(v16f (&S)[NT], int k, v16f v) {
+#pragma unroll
+  for (int i = 0; i < NT; i++)
+    if (k == i) {
+      S[i] = v;
+      asm volatile("" : "+v"(S[i]));
+    }
+}
+
+// LDS: q [HD][16] fp32, then per wave a K tile (up to 64 elements of 64 rows,
+// fp16), later the probabilities of one of its tiles [64][16]
+constexpr int kMmWaves = 8;
+constexpr int kMmWaveLds = 8192;
+static_assert(kPfTile * kMmTok * 4 <= kMmWaveLds, "a tile's probabilities");
+template <int HD>
+constexpr size_t mm_lds_bytes() {
+  return (size_t)kMmTok * HD * 4 + kMmWaves * kMmWaveLds;
+}
+
+template <int HD, int NT>
+__global__ __launch_bounds__(kMmWaves * 64, NT > 4 ? 2 : 4) void attn_prefill_mm_kernel(AttnArgs a, int ngroups) {
+  constexpr int T = kMmTok, NW = kMmWaves, NTH = NW * 64;
+  constexpr int DG = HD / 16;                       // groups of 16 output elements
+  constexpr int KH = HD < 64 ? HD : 64;             // elements of a K row staged at a time
+  constexpr int CPR = KH / 8, RPI = 64 / CPR;       // 16-byte chunks per staged row, rows per load instruction
+  static_assert(NW >= DG, "a wave per 16 output elements");
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float *qt = lds;                                      // q as [HD][16]
+  char *wbuf = reinterpret_cast<char *>(lds + T * HD);  // kMmWaveLds bytes per wave
+  __shared__ uint64_t etab[32];
+  __shared__ float s_max[NW][T];
+  __shared__ double s_sum[NW][T];
+
+  const int t = threadIdx.x, lane = t & 63, lr = lane & 15, lq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int h = blockIdx.x, kvh = h * a.KVH / a.H;
+  const int m0 = (ngroups - 1 - (int)blockIdx.y) * T;  // longest key ranges first
+  const int slot = ld_uniform(a.slot + m0);
+  const int pos_first = ld_uniform(a.pos + m0), pos_hi = ld_uniform(a.pos + min(m0 + T - 1, a.M - 1));
+  const int lo0 = a.window > 0 ? max(0, pos_first - a.window + 1) : 0;
+  const int lo_hi = a.window > 0 ? max(0, pos_hi - a.window + 1) : 0;
+  const int ntile = (pos_hi - lo0) / kPfTile + 1;
+  if (t < 32) etab[t] = ec_exp2_32[t];
+  const size_t cbase = (size_t)slot * a.C * a.kv + (size_t)kvh * HD;
+  const uint16_t *Kc = a.kc + cbase, *Vc = a.vc + cbase;
+
+  for (int e = t; e < T * HD / 4; e += NTH) {
+    const int r = e % T, c4 = e / T;
+    const float4 v = *reinterpret_cast<const float4 *>(a.q + (size_t)min(m0 + r, a.M - 1) * a.ldq + (size_t)h * HD + 4 * c4);
+    float *dst = qt + 4 * c4 * T + r;
+    dst[0] = v.x;
+    dst[T] = v.y;
+    dst[2 * T] = v.z;
+    dst[3 * T] = v.w;
+  }
+  __syncthreads();
+
+  // whether every token takes every position of the tile that starts at p0
+  auto whole = [&](int p0) { return p0 >= lo_hi && p0 + kPfTile - 1 <= pos_first; };
+  // whether this lane's token r takes position p (tokens past the prompt, which
+  // are not stored, take those of the last one)
+  auto takes = [&](int p, int r) {
+    const int tp = pos_first + min(4 * lq + r, pos_hi - pos_first);
+    const int tl = a.window > 0 ? max(0, tp - a.window + 1) : 0;
+    return (unsigned)(p - tl) <= (unsigned)(tp - tl);
+  };
+
+  // ---- scores ----
+  v16f S[NT];
+  float mx[4] = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+  const int nk = w < ntile ? (ntile - 1 - w) / NW + 1 : 0;  // this wave's tiles
+  // chunk c of row r of a staged tile is at chunk c ^ swz(r) of the row: 8
+  // consecutive rows' 16-byte reads of one chunk fall on distinct banks
+  auto swz = [](int r) { return CPR == 8 ? r & 7 : (r >> 1) & 3; };
+  const int krow = lane / CPR, kchk = lane % CPR;
+  const char *kld = wbuf + w * kMmWaveLds + lane * (2 * KH);
+  const int ksw = 16 * swz(lane);
+#pragma unroll 1
+  for (int k = 0; k < nk; k++) {
+    const int tile = k * NW + w, p0 = lo0 + kPfTile * tile;
+    v16f acc = {0};
+#pragma unroll 1
+    for (int e0 = 0; e0 < HD; e0 += KH) {
+      // the tile's rows, whole 128-byte lines per instruction, through this
+      // wave's part of the LDS: a lane reads its position's row (no barrier:
+      // one wave's LDS operations are in order)
+      {
+        v4u kr[CPR];
+#pragma unroll
+        for (int i = 0; i < CPR; i++) {
+          const int p = min(p0 + RPI * i + krow, pos_hi);
+          kr[i] = *reinterpret_cast<const v4u *>(Kc + (size_t)p * a.kv + e0 + 8 * kchk);
+        }
+#pragma unroll
+        for (int i = 0; i < CPR; i++) {
+          const int r = RPI * i + krow;
+          *reinterpret_cast<v4u *>(wbuf + w * kMmWaveLds + r * (2 * KH) + 16 * (kchk ^ swz(r))) = kr[i];
+        }
+      }
+      const float *qa = qt + e0 * T + lane;
+      v4u kc = *reinterpret_cast<const v4u *>(kld + (0 ^ ksw));
+      float aq = qa[0];
+#pragma unroll
+      for (int c = 0; c < CPR; c++) {
+        const v4u kn = *reinterpret_cast<const v4u *>(kld + ((16 * (c + 1 < CPR ? c + 1 : c)) ^ ksw));
+        const float a1 = qa[(2 * c + 1) * 64], a2 = qa[(2 * (c + 1 < CPR ? c + 1 : c)) * 64];
+        const uint32_t hv[4] = {kc.x, kc.y, kc.z, kc.w};
+        // the asm statements keep the compiler from forming all products first
+#define MM_STEP(e, av, ab)                                                                             \
+  {                                                                                                    \
+    uint32_t hw = hv[(e) / 2];                                                                         \
+    asm volatile("" : "+v"(acc), "+v"(hw));                                                            \
+    acc += mm_bcast<ab>(av, h2f((uint16_t)((e) & 1 ? hw >> 16 : hw & 0xffffu)));                       \
+  }
+        MM_STEP(0, aq, 0)
+        MM_STEP(1, aq, 1)
+        MM_STEP(2, aq, 2)
+        MM_STEP(3, aq, 3)
+        MM_STEP(4, a1, 0)
+        MM_STEP(5, a1, 1)
+        MM_STEP(6, a1, 2)
+        MM_STEP(7, a1, 3)
+#undef MM_STEP
+        aq = a2;
+        kc = kn;
+      }
+    }
+    const bool wh = whole(p0);
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float s = (float)((double)acc[4 * b + r] * a.inv_hd);
+        if (wh || takes(p0 + 16 * b + lr, r)) mx[r] = fmaxf(mx[r], s);
+        else s = -__builtin_inff();
+        acc[4 * b + r] = s;
+      }
+    mm_put<NT>(S, k, acc);
+  }
+
+  // ---- softmax: maximum, exponentials and their sum ----
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    float v = mx[r];
+    v = fmaxf(v, dpp_mov<0xB1>(v));
+    v = fmaxf(v, dpp_mov<0x4E>(v));
+    v = fmaxf(v, dpp_mov<0x141>(v));
+    v = fmaxf(v, dpp_mov<0x140>(v));
+    if (lr == 0) s_max[w][4 * lq + r] = v;
+  }
+  __syncthreads();
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    mx[r] = s_max[0][4 * lq + r];
+#pragma unroll
+    for (int i = 1; i < NW; i++) mx[r] = fmaxf(mx[r], s_max[i][4 * lq + r]);
+  }
+#pragma unroll 1
+  for (int k = 0; k < nk; k++) {
+    v16f v = mm_get<NT>(S, k);
+    const int p0 = lo0 + kPfTile * (k * NW + w);
+    const bool wh = whole(p0);
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      // four exponentials at a time (more exceed the registers): the table
+      // reads of all four in flight together
+      double er[4];
+      uint64_t ki[4], et[4];
+      float x[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        x[r] = v[4 * b + r] - mx[r];
+        ki[r] = ec_expf_head(x[r], &er[r]);
+        et[r] = etab[ki[r] % 32];
+      }
+      asm volatile("" : "+v"(v), "+v"(et[0]), "+v"(et[1]), "+v"(et[2]), "+v"(et[3]));
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float e = ec_expf_tail(x[r], er[r], ki[r], et[r]);
+        if (!wh && !takes(p0 + 16 * b + lr, r)) e = 0.0f;
+        v[4 * b + r] = e;
+        sum[r] += (double)e;
+      }
+    }
+    mm_put<NT>(S, k, v);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    double v = sum[r];
+    v = v + dpp_mov<0xB1>(v);
+    v = v + dpp_mov<0x4E>(v);
+    v = v + dpp_mov<0x141>(v);
+    v = v + dpp_mov<0x140>(v);
+    if (lr == 0) s_sum[w][4 * lq + r] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    double v = s_sum[0][4 * lq + r];
+#pragma unroll
+    for (int i = 1; i < NW; i++) v += s_sum[i][4 * lq + r];
+    sum[r] = 1.0 / v;
+  }
+
+  // ---- output ----
+  // this lane's element of position p0 + 4 s + lane / 16, from the cache (two
+  // bytes per lane, 32 of a row: the waves' loads of a row share its line);
+  // rows past pos_hi read as zero (their products are masked)
+  v4f o = {0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr int NS = kPfTile / 8;  // steps of four positions per half tile
+  uint16_t vr[NS], vn[NS];
+  const uint64_t vbase = (uint64_t)(uintptr_t)(Vc + (size_t)lo0 * a.kv);
+  const uint32_t vlo = __builtin_amdgcn_readfirstlane((uint32_t)vbase),
+                 vhi = __builtin_amdgcn_readfirstlane((uint32_t)(vbase >> 32));
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(uintptr_t)(((uint64_t)vhi << 32) | vlo), 0, ((pos_hi - lo0) * a.kv + HD) * 2, 0x00020000);
+  int voff = 2 * (lq * a.kv + 16 * (w < DG ? w : 0) + lr);  // the whole offset: the range check covers it
+  auto vload = [&]() {
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      vn[s] = __builtin_amdgcn_raw_buffer_load_b16(vrs, voff, 0, 0);
+      voff += 8 * a.kv;
+    }
+  };
+  vload();
+#pragma unroll 1
+  for (int t0 = 0; t0 < ntile; t0 += NW) {
+    __syncthreads();  // the previous NW tiles' probabilities are consumed
+    if (t0 + w < ntile) {
+      const v16f v = mm_get<NT>(S, t0 / NW);
+      float *dst = reinterpret_cast<float *>(wbuf + w * kMmWaveLds) + lr * T + 4 * lq;
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        float4 p;
+        p.x = (float)((double)v[4 * b] * sum[0]);
+        p.y = (float)((double)v[4 * b + 1] * sum[1]);
+        p.z = (float)((double)v[4 * b + 2] * sum[2]);
+        p.w = (float)((double)v[4 * b + 3] * sum[3]);
+        *reinterpret_cast<float4 *>(dst + 16 * b * T) = p;
+      }
+    }
+    __syncthreads();
+    if (w >= DG) continue;
+#pragma unroll 1
+    for (int half = 0; half < 2 * min(NW, ntile - t0); half++) {
+      const int p0 = lo0 + kPfTile * t0 + kPfTile / 2 * half;
+      const float *pa = reinterpret_cast<const float *>(wbuf + (half >> 1) * kMmWaveLds) + (half & 1) * (64 * NS) + lane;
+      // the next half tile's values are loaded while this one's are used
+#pragma unroll
+      for (int s = 0; s < NS; s++) vr[s] = vn[s];
+      vload();
+      // a step's probabilities are read four steps ahead, its products formed one ahead
+      auto sums = [&](auto masked) {
+        float fa[NS];
+#pragma unroll
+        for (int s = 0; s < 4; s++) fa[s] = pa[64 * s];
+        v16f pn = __builtin_amdgcn_mfma_f32_16x16x1f32(fa[0], h2f(vr[0]), v16f{0}, 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          v16f pc = pn;
+          if (s + 4 < NS) fa[s + 4] = pa[64 * (s + 4)];
+          if (s + 1 < NS) {
+            asm volatile("" : "+v"(o), "+v"(fa[s + 1]));
+            pn = __builtin_amdgcn_mfma_f32_16x16x1f32(fa[s + 1], h2f(vr[s + 1]), v16f{0}, 0, 0, 0);
+          }
+          if constexpr (masked.value) {
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                if (!takes(p0 + 4 * s + b, r)) pc[4 * b + r] = -0.0f;
+          }
+#pragma unroll
+          for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = o[r] + pc[4 * b + r];
+        }
+      };
+      if (p0 >= lo_hi && p0 + kPfTile / 2 - 1 <= pos_first) sums(std::false_type{});
+      else if (p0 <= pos_hi) sums(std::true_type{});
+    }
+  }
+  if (w < DG) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = m0 + 4 * lq + r;
+      if (m < a.M) a.out[(size_t)m * a.ldo + (size_t)h * HD + 16 * w + lr] = o[r];
+    }
+  }
+}
+
+// positions that one block of 16 tokens reads
+int mm_span(const AttnArgs &a) {
+  int r = a.max_npos;
+  if (a.window > 0 && a.window + kMmTok - 1 < r) r = a.window + kMmTok - 1;
+  return r;
+}
+// the most positions whose scores the kernel's registers hold
+constexpr int kMmMaxSpan = 8 * kMmWaves * kPfTile;
+
+template <int HD, int NT>
+void launch_mm(const AttnArgs &a, hipStream_t st) {
+  const int ngroups = (a.M + kMmTok - 1) / kMmTok;
+  klaunch((attn_prefill_mm_kernel<HD, NT>), dim3(a.H, ngroups), dim3(kMmWaves * 64), mm_lds_bytes<HD>(), st, a, ngroups);
+}
+
+// Whether the matrix-core kernel takes a prompt: its scores fit the registers,
+// and at head_dim 128, where the other kernel spreads a short prompt over twice
+// the blocks (8 tokens each), it has at least 192 blocks: 12 heads of 128,
+// 128 tokens (96 blocks) 30.2 us there, 34.2 us here; 256 tokens (192 blocks)
+// 38.5 and 38.1 us; 64 tokens after 1500 (48 blocks) 99.6 and 111.5 us.  At
+// head_dim 64 it is faster from 16 tokens (27.7 -> 27.1 us) on.
+bool mm_takes(const AttnArgs &a) {
+  if (mm_span(a) > kMmMaxSpan) return false;
+  return a.hd != 128 || (long)a.H * ((a.M + kMmTok - 1) / kMmTok) >= 192;
+}
+
+// by the longest span: the fewest score registers that hold it (up to 2048
+// positions two blocks share a CU, beyond that one)
+template <int HD>
+void launch_mm_any(const AttnArgs &a, hipStream_t st) {
+  const int n = mm_span(a);
+  if (n <= kMmWaves * kPfTile) launch_mm<HD, 1>(a, st);
+  else if (n <= 4 * kMmWaves * kPfTile) launch_mm<HD, 4>(a, st);
+  else launch_mm<HD, 8>(a, st);
 }
 
 // score slots per token: the positions one block reads, window-bounded
@@ -758,37 +756,30 @@ size_t pf_lds_bytes(const AttnArgs &a, int qb) {
   return ((size_t)(kPfTile + 4) * (a.hd + 4) + (size_t)qb * pf_nsc(a, qb) + 4) * sizeof(float) + 256;
 }
 
-// block shapes, largest first: (waves, tokens per wave)
-constexpr int kPfShapes[3][2] = {{8, 2}, {8, 1}, {4, 1}};
+// waves (of one token) per block, largest first
+constexpr int kPfShapes[2] = {8, 4};
 
 int pf_pick(const AttnArgs &a, int max_lds) {
-  for (int i = 0; i < 3; i++) {
-    if (a.hd == 128 && kPfShapes[i][1] > 1) continue;  // two q rows of 128 do not fit the registers
-    if (pf_lds_bytes(a, kPfShapes[i][0] * kPfShapes[i][1]) <= (size_t)max_lds) return i;
-  }
+  for (int i = 0; i < 2; i++)
+    if (pf_lds_bytes(a, kPfShapes[i]) <= (size_t)max_lds) return i;
   return -1;
 }
 
 // grid (head, token group): consecutive block ids, which the dispatcher deals
 // out to the 8 XCDs in turn, spread every head over every XCD; one slot's K/V
 // of all KV heads fits each XCD's L2 at the prefill lengths of the models
-template <int HD, int NW, int QW>
+template <int HD, int NW>
 void launch_pf(const AttnArgs &a, hipStream_t st) {
-  const int ngroups = (a.M + NW * QW - 1) / (NW * QW);
+  const int ngroups = (a.M + NW - 1) / NW;
   const dim3 grid(a.H, ngroups);
-  klaunch((attn_prefill_kernel<HD, NW, QW>), grid, dim3(NW * 64), pf_lds_bytes(a, NW * QW) - 256, st, a,
-          ngroups, pf_nsc(a, NW * QW));
+  klaunch((attn_prefill_kernel<HD, NW, 1>), grid, dim3(NW * 64), pf_lds_bytes(a, NW) - 256, st, a, ngroups,
+          pf_nsc(a, NW));
 }
 
 template <int HD>
 void launch_hd(const AttnArgs &a, int shape, hipStream_t st) {
-  if (shape == 0) {
-    if constexpr (HD != 128) launch_pf<HD, 8, 2>(a, st);
-  } else if (shape == 1) {
-    launch_pf<HD, 8, 1>(a, st);
-  } else {
-    launch_pf<HD, 4, 1>(a, st);
-  }
+  if (shape == 0) launch_pf<HD, 8>(a, st);
+  else launch_pf<HD, 4>(a, st);
 }
 
 }  // namespace
@@ -796,11 +787,17 @@ void launch_hd(const AttnArgs &a, int shape, hipStream_t st) {
 bool attention_prefill_ok(const AttnArgs &a, int max_lds) {
   if (!(a.hd == 32 || a.hd == 64 || a.hd == 128) || !attn_vec(a.hd, a.kv) || a.fuse_kv || a.M < 1) return false;
   if (a.ldq % 4 || ((uintptr_t)a.q & 15u)) return false;  // q rows read as float4
-  return pf_pick(a, max_lds) >= 0;
+  return mm_takes(a) || pf_pick(a, max_lds) >= 0;
 }
 
 hipError_t attention_prefill(const AttnArgs &a, int max_lds, hipStream_t st) {
   if (!attention_prefill_ok(a, max_lds)) return hipErrorInvalidValue;
+  if (mm_takes(a)) {
+    if (a.hd == 64) launch_mm_any<64>(a, st);
+    else if (a.hd == 128) launch_mm_any<128>(a, st);
+    else launch_mm_any<32>(a, st);
+    return hipGetLastError();
+  }
   const int shape = pf_pick(a, max_lds);
   if (a.hd == 64) launch_hd<64>(a, shape, st);
   else if (a.hd == 128) launch_hd<128>(a, shape, st);

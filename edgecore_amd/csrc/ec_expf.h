@@ -42,30 +42,35 @@ EC_EXPF_TABLE uint64_t ec_exp2_32[32] = {
     0x3fef5818dcfba487ull, 0x3fef7c97337b9b5full, 0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-/* tab: the 32 entries of ec_exp2_32, wherever the caller keeps a copy
- * (kernels stage them in LDS so the lookup does not wait on memory) */
-EC_EXPF_FN float ec_expf_tab(float x, const uint64_t *tab)
+/* The argument's part, up to the table: x*32/ln2 = k + r.  Returns k's bits
+ * (the table index is their low five). */
+EC_EXPF_FN uint64_t ec_expf_head(float x, double *r)
 {
     const double inv_ln2_n = 0x1.71547652b82fep+0 * 32.0;
     const double shift = 0x1.8p+52;
-    const double c0 = 0x1.c6af84b912394p-5 / 32768.0; /* / 32^3 */
-    const double c1 = 0x1.ebfce50fac4f3p-3 / 1024.0;  /* / 32^2 */
-    const double c2 = 0x1.62e42ff0c52d6p-1 / 32.0;
-    uint32_t ux;
-    memcpy(&ux, &x, 4);
-    const uint32_t abstop = (ux >> 20) & 0x7ffu;
-    /* the main path for every input; glibc's special cases (|x| >= 88, inf,
-     * nan) replace its result below by selects, in glibc's order of
-     * precedence, so that a wave takes no branch (the main path of inf or
-     * nan yields some value, and its table index stays in 0..31) */
     const double xd = (double)x;
     const double z = inv_ln2_n * xd;
     double kd = z + shift;
     uint64_t ki;
     memcpy(&ki, &kd, 8);
     kd -= shift;
-    const double r = __builtin_fma(inv_ln2_n, xd, -kd);
-    uint64_t t = tab[ki % 32];
+    *r = __builtin_fma(inv_ln2_n, xd, -kd);
+    return ki;
+}
+
+/* The result from the table's entry t = tab[ki % 32].  The main path for every
+ * input; glibc's special cases (|x| >= 88, inf, nan) replace its result by
+ * selects, in glibc's order of precedence, so that a wave takes no branch (the
+ * main path of inf or nan yields some value, and its table index stays in
+ * 0..31). */
+EC_EXPF_FN float ec_expf_tail(float x, double r, uint64_t ki, uint64_t t)
+{
+    const double c0 = 0x1.c6af84b912394p-5 / 32768.0; /* / 32^3 */
+    const double c1 = 0x1.ebfce50fac4f3p-3 / 1024.0;  /* / 32^2 */
+    const double c2 = 0x1.62e42ff0c52d6p-1 / 32.0;
+    uint32_t ux;
+    memcpy(&ux, &x, 4);
+    const uint32_t abstop = (ux >> 20) & 0x7ffu;
     t += ki << 47;
     double s;
     memcpy(&s, &t, 8);
@@ -80,6 +85,15 @@ EC_EXPF_FN float ec_expf_tab(float x, const uint64_t *tab)
     res = abstop >= 0x7f8u ? x + x : res;             /* inf or nan */
     res = ux == 0xff800000u ? 0.0f : res;             /* -inf */
     return res;
+}
+
+/* tab: the 32 entries of ec_exp2_32, wherever the caller keeps a copy
+ * (kernels stage them in LDS so the lookup does not wait on memory) */
+EC_EXPF_FN float ec_expf_tab(float x, const uint64_t *tab)
+{
+    double r;
+    const uint64_t ki = ec_expf_head(x, &r);
+    return ec_expf_tail(x, r, ki, tab[ki % 32]);
 }
 
 EC_EXPF_FN float ec_expf_ref(float x) { return ec_expf_tab(x, ec_exp2_32); }

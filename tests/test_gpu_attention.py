@@ -113,3 +113,35 @@ def test_attention_dev_rejects_bad_arguments():
         ec.attention_dev(q, kc, vc, [0, 1, 3, 4], [0, 0, 0, 0], H, KVH, path=0)  # not consecutive
     with pytest.raises(ec.EdgeCoreError):
         ec.attention_dev(q, kc, vc, [0, 1, 2, 3], [0, 0, 1, 0], H, KVH)          # slot outside the cache
+
+
+# the matrix-core prefill kernel: 16 tokens per block (1, 15, 17, 33 of them),
+# 64-position tiles, 1 (span 512), 4 (2048) and 8 (4096) of them per wave, and
+# past that the other kernel; head_dim 128 takes it from 192 blocks on
+@pytest.mark.parametrize("H,KVH,hd,M,p0,window", [
+    (2, 1, 64, 1, 0, 0), (2, 1, 64, 15, 49, 0), (2, 2, 64, 17, 48, 0), (3, 1, 64, 33, 479, 0), (2, 1, 64, 33, 480, 0),
+    (2, 1, 64, 20, 2028, 0), (2, 1, 64, 21, 2028, 0), (1, 1, 64, 16, 4080, 0), (1, 1, 64, 16, 4081, 0),
+    (2, 1, 64, 40, 700, 1), (2, 1, 64, 70, 0, 497), (2, 1, 64, 70, 430, 498), (2, 1, 32, 33, 500, 0),
+    (2, 2, 32, 17, 2100, 0), (96, 8, 128, 31, 0, 0), (96, 8, 128, 32, 490, 0), (96, 8, 128, 17, 1000, 300),
+    (96, 8, 128, 17, 2040, 0)])
+def test_prefill_matrix_core_edges(H, KVH, hd, M, p0, window):
+    rng, q, kc, vc = _case(M + p0 + hd + window, M, H, KVH, hd, p0 + M, 2)
+    pos, sl = p0 + np.arange(M), np.ones(M)
+    got = ec.attention_dev(q, kc, vc, pos, sl, H, KVH, window=window, path=0)
+    want = oracle.attention_rows(q, kc, vc, pos, sl, H, KVH, window=window)
+    _check(got, want, np.arange(M))
+
+
+@pytest.mark.parametrize("hd,H", [(64, 2), (128, 96)])
+def test_prefill_value_not_finite_outside_a_tokens_range(hd, H):
+    """An infinity in the last position's value reaches that position's token
+    alone, and one before a window no token inside it."""
+    M, KVH, window = 40, 2, 20
+    _, q, kc, vc = _case(hd, M, H, KVH, hd, M, 1)
+    vc[0, M - 1] = 0x7C00
+    vc[0, 0] = 0xFC00
+    pos, sl = np.arange(M), np.zeros(M)
+    got = ec.attention_dev(q, kc, vc, pos, sl, H, KVH, window=window, path=0)
+    want = oracle.attention_rows(q, kc, vc, pos, sl, H, KVH, window=window)
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    _check(got, want, np.arange(window, M - 1))
