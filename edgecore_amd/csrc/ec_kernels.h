@@ -90,6 +90,11 @@ hipError_t gemv_i8_fused(const GemvArgs &a, int epi, int pro, hipStream_t s);
 hipError_t gemv_f16_fused(const GemvArgs &a, int epi, int pro, hipStream_t s);
 hipError_t gemv_bf16_fused(const GemvArgs &a, int epi, int pro, hipStream_t s);
 hipError_t gemv_generic(const GemvArgs &a, int wt, int epi, hipStream_t s);
+// 16-bit weights, fp32 rows, plain store: a few activation rows in registers
+// (gemv_regs.hip); K up to 1536.  gemv_regs_faster: than the fused GEMV.
+bool gemv_regs_ok(const GemvArgs &a, int wt);
+bool gemv_regs_faster(const GemvArgs &a, int wt);
+hipError_t gemv_regs(const GemvArgs &a, int wt, hipStream_t s);
 // int8 matrix-core GEMM (gemm_mfma.hip) for M >= kGemmMinM: int8 A rows with
 // scales as (PRO_I8 input), every epilogue but argmax candidates; the floats
 // equal the vector GEMV's for the same rows.  gemm_i8_ok: shape and alignment

@@ -500,6 +500,10 @@ static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int 
     EC_LAUNCH("gemm_w16", bytes, gemm_w16(a, wt, EPI_STORE, g_w16_parts, ldp, g_w16_rs, g_stream));
     return 0;
   }
+  if (gemv_regs_faster(a, wt)) {
+    EC_LAUNCH("gemv_w16", bytes, gemv_regs(a, wt, g_stream));
+    return 0;
+  }
   EC_LAUNCH("gemv_w16", bytes, gemv_any(a, wt, EPI_STORE, PRO_F32, g_stream));
   return 0;
 }
@@ -1351,6 +1355,15 @@ static const char *gemm_family(const char *fam) {
   return "gemm_i8";
 }
 
+// A language-model head of 2 to 15 rows: the norm as its own launch (about 4
+// us), then the rows in registers, where that outweighs the fused GEMV's norm.
+// 65536 outputs: 8 rows x 8192 13 us fused, 7 + 4 us here; 2 x 50257 (K = 768)
+// 20.7 and 15.9 + 4 us.
+static bool lm_head_regs(const GemvArgs &a, int wt, int epi, int pro) {
+  return epi == EPI_STORE && (pro == PRO_RMS || pro == PRO_LN) && a.M < kGemmMinM && (long)a.M * a.N >= 65536 &&
+         a.N >= 8192 && gemv_regs_faster(a, wt);
+}
+
 static int linear(GPT2 *g, DevModel *d, const char *fam, GemvArgs a, int wt, int epi, int pro, hipStream_t s) {
   const double bytes = gemv_bytes(wt, pro, epi, a.M, a.K, a.N, a.ws != nullptr, a.bias != nullptr);
   if (wt == WT_I8 && g_use_mfma && a.M >= kGemmMinM) {
@@ -1400,6 +1413,14 @@ static int linear(GPT2 *g, DevModel *d, const char *fam, GemvArgs a, int wt, int
     EC_LAUNCH("split16", 4.0 * a.M * a.K * (1.0 + w16_parts(wt) / 2.0),
               split_rows16(q, wt, d->ah, d->ah_ld, d->ahs, s));
     EC_LAUNCH(gemm_family(fam), bytes, gemm_w16_parts(q, wt, epi, 0, d->ah, d->ah_ld, d->ahs, s));
+    return 0;
+  }
+  if (lm_head_regs(a, wt, epi, pro)) {
+    EC_LAUNCH("norm", 8.0 * a.M * a.K,
+              norm_rows((const float *)a.A, a.M, a.K, a.gamma, a.beta, g->eps, d->h, a.K, nullptr, 0, nullptr, s));
+    a.A = d->h;
+    a.lda = a.K;
+    EC_LAUNCH(fam, bytes, gemv_regs(a, wt, s));
     return 0;
   }
   if (a.pmax_out == d->pmax_ff) d->ff_pmax = false;  // the paths below leave the partial maxima unwritten
@@ -1772,7 +1793,7 @@ static int enqueue_forward(GPT2 *g, DevModel *d, int M, int lm_from, bool distin
     // argmax to argmax_rows; the fused GEMV keeps per-block candidates
     const bool mfma = g_use_mfma && rows >= kGemmMinM && rows <= d->ah_rows && E <= d->ah_ld &&
                       gemm_w16_ok(a, lwt, EPI_STORE);
-    const bool fused = !mfma && gemv_vector_ok(a, lwt, pro_norm);
+    const bool fused = !mfma && !lm_head_regs(a, lwt, EPI_STORE, pro_norm) && gemv_vector_ok(a, lwt, pro_norm);
     if (argmax && fused) a.cand = d->cand;
     if ((r = linear(g, d, "gemv_lmhead", a, lwt, EPI_STORE, pro_norm, s))) return r;
     if (argmax) {
