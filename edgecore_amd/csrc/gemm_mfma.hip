@@ -149,8 +149,12 @@ __device__ unsigned gm_cnt[kGmMaxTiles];
 
 // A: [M * NP][lda] elements (row m's part p at row m * NP + p), as: per-row
 // scale (int8 quantization scale, or the split's 2^e; 1 for bf16)
-template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false>
+// RAG: rows that may end inside a 16-byte chunk, operands at any address, the
+// check for values that are not finite (a form of its own: the others ran 1-2%
+// slower with its branches in them)
+template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool RAG = false>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
+  static_assert(!(RAG && DL), "the direct-to-LDS form takes whole aligned stages");
   using Op = MfmaOp<OP>;
   using Acc = typename Op::Acc;
   constexpr int NP = Op::NP;
@@ -199,7 +203,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   float e_old[RES ? TI : 1][RES ? JO : 1][4];
   {
     // N*K >= 4N bytes: valid for every column index (weights at odd addresses: the output's row 0)
-    const float *stand = ((uintptr_t)a.W & 3) ? a.out : (const float *)a.W;
+    const float *stand = RAG && ((uintptr_t)a.W & 3) ? a.out : (const float *)a.W;
     const float *wsp = a.ws ? a.ws : stand, *bvp = a.bias ? a.bias : stand;
     const float *ws2p = (SWI && a.ws2) ? a.ws2 : stand;
 #pragma unroll
@@ -261,13 +265,17 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   auto load = [&](int k0) {
     kl = k0;
 #pragma unroll
-    for (int j = 0; j < ACH; j++)
-      ra[j] = ld16(arow[j] + min(k0 + 16 * acol[j], KB - 16));
+    for (int j = 0; j < ACH; j++) {
+      const int8_t *p = arow[j] + min(k0 + 16 * acol[j], KB - 16);
+      ra[j] = RAG ? ld16(p) : *reinterpret_cast<const v4i *>(p);
+    }
 #pragma unroll
-    for (int j = 0; j < BCH; j++)
-      rb[j] = ld16(brow[j] + min(k0 + 16 * bcol[j], KB - 16));
+    for (int j = 0; j < BCH; j++) {
+      const int8_t *p = brow[j] + min(k0 + 16 * bcol[j], KB - 16);
+      rb[j] = RAG ? ld16(p) : *reinterpret_cast<const v4i *>(p);
+    }
   };
-  const bool rag = KB & 15;  // the row ends inside a chunk
+  const bool rag = RAG && (KB & 15);  // the row ends inside a chunk
   auto store = [&](int buf) {
     const v4i z = {0, 0, 0, 0};
     if (rag) {
@@ -482,7 +490,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     if (t == 0) __hip_atomic_store(&gm_cnt[tl], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  if constexpr (!I8) {
+  if constexpr (!I8 && RAG) {
     if (a.Af) {  // uniform
       bool bad = false;
 #pragma unroll
@@ -602,7 +610,9 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   // (24 tiles of 32 x 128 over 48 stages of K) ran each tile's whole K on
   // one CU while 232 CUs idled
   const bool dl = EC_GEMM_DL && (a.K * MfmaOp<OP>::EB) % kBK == 0 && (a.lda * MfmaOp<OP>::EB) % kBK == 0 &&
-                  aligned16(a.A) && aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2));
+                  aligned16(a.A) && aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2)) && !a.Af;
+  const bool rag = a.Af || (a.K * MfmaOp<OP>::EB) % 16 || (a.lda * MfmaOp<OP>::EB) % 16 || !aligned16(a.A) ||
+                   !aligned16(a.W) || (EPI == EPI_SWIGLU && !aligned16(a.W2));
   const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM) : 1;
   const dim3 grid(8 * ((T + 7) / 8), ks);
   if constexpr (BM == 32) {
@@ -628,6 +638,9 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
     klaunch((gemm_mfma_kernel<OP, BM, EPI, true, l3 <= 158 * 1024 ? 3 : 2>), grid, dim3(256),
             gemm_lds_bytes<OP, BM, true, l3 <= 158 * 1024 ? 3 : 2>(), s, a);
   else if (dl) klaunch((gemm_mfma_kernel<OP, BM, EPI, true>), grid, dim3(256), gemm_lds_bytes<OP, BM, true>(), s, a);
+  else if (rag)
+    klaunch((gemm_mfma_kernel<OP, BM, EPI, false, 2, false, true>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s,
+            a);
   else klaunch((gemm_mfma_kernel<OP, BM, EPI, false>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s, a);
   return hipGetLastError();
 }
