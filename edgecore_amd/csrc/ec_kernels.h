@@ -95,11 +95,16 @@ hipError_t gemv_generic(const GemvArgs &a, int wt, int epi, hipStream_t s);
 bool gemv_regs_ok(const GemvArgs &a, int wt);
 bool gemv_regs_faster(const GemvArgs &a, int wt);
 hipError_t gemv_regs(const GemvArgs &a, int wt, hipStream_t s);
-// int8 matrix-core GEMM (gemm_mfma.hip) for M >= kGemmMinM: int8 A rows with
+// int8 matrix-core GEMM (gemm_mfma.hip) for M >= kGemmMinMI8: int8 A rows with
 // scales as (PRO_I8 input), every epilogue but argmax candidates; the floats
 // equal the vector GEMV's for the same rows.  gemm_i8_ok: shape and alignment
 // (K % 16, lda % 16, 16-byte aligned A / W / W2).
 constexpr int kGemmMinM = 16;
+// int8 rows from which the skinny form is the faster one (the fused GEMV takes
+// row tiles of 8 above 4): 6 rows, K x N: 896 x 896 5.7 -> 4.6 us, 896 x 9728
+// 6.2 -> 5.4, 1536 x 17920 17.2 -> 11.0, 8960 x 1536 10.1 -> 8.0; 4 rows of
+// 4864 x 896 5.3 there, 6.6 here
+constexpr int kGemmMinMI8 = 5;
 bool gemm_i8_ok(const GemvArgs &a, int epi);
 // any K from 16 and any alignment (unaligned 16-byte loads): what the
 // launchers below take; gemm_i8_ok shapes run faster

@@ -62,7 +62,7 @@ static hipDeviceProp_t g_prop;
 static int g_max_lds = 65536;
 // replay the single-token greedy step as a HIP graph (EDGECORE_GRAPHS=0 turns it off)
 static bool g_use_graphs = true;
-// int8 linears with kGemmMinM rows or more on the matrix cores
+// int8 linears with kGemmMinMI8 rows or more (16-bit: kGemmMinM) on the matrix cores
 // (EDGECORE_MFMA=0: the vector GEMV for every M)
 static bool g_use_mfma = true;
 
@@ -399,7 +399,7 @@ extern "C" int ec_gemm_int8_dev(float *C, const int8_t *A, const float *a_scale,
   if (!C || !a_scale || (K > 0 && (!A || !B))) return set_err(-1, "gemm_int8: null pointer");
   GemvArgs a{A, K, a_scale, nullptr, nullptr, 0.0, B, nullptr, b_scale, nullptr, bias, C, N, M, K, N, nullptr};
   const double bytes = gemv_bytes(WT_I8, PRO_I8, EPI_STORE, M, K, N, b_scale, bias);
-  if (g_use_mfma && M >= kGemmMinM && gemm_i8_ok(a, EPI_STORE)) {
+  if (g_use_mfma && M >= kGemmMinMI8 && gemm_i8_ok(a, EPI_STORE)) {
     if (M <= 32) {
       EC_LAUNCH("gemm_i8", bytes, gemm_i8_skinny(a, EPI_STORE, 0, g_stream));
     } else {
@@ -737,7 +737,7 @@ struct DevModel {
   float *ahs = nullptr;
   float *logits = nullptr;
   float *att_sc = nullptr;  // decode attention scores [batch_cap][H][eff_ctx] (long contexts)
-  // Batched decode (16-32 tokens) with the activation quantization of the o
+  // Batched decode (5-32 tokens) with the activation quantization of the o
   // and down projections inside their skinny GEMMs (EDGECORE_FUSEQ=0 at load
   // turns it off): partial row maxima of the attention output [32][4 H] and
   // of the FFN activation [32][ceil(F / 16)], written by the attention and
@@ -1366,7 +1366,7 @@ static bool lm_head_regs(const GemvArgs &a, int wt, int epi, int pro) {
 
 static int linear(GPT2 *g, DevModel *d, const char *fam, GemvArgs a, int wt, int epi, int pro, hipStream_t s) {
   const double bytes = gemv_bytes(wt, pro, epi, a.M, a.K, a.N, a.ws != nullptr, a.bias != nullptr);
-  if (wt == WT_I8 && g_use_mfma && a.M >= kGemmMinM) {
+  if (wt == WT_I8 && g_use_mfma && a.M >= kGemmMinMI8) {
     // batched decode: the quantization inside the skinny GEMM, from the
     // producer's partial row maxima
     if (pro == PRO_QUANT && a.pmax && (a.pmax != d->pmax_ff || d->ff_pmax) && gemm_i8_skinny_q_ok(a, epi)) {
@@ -1648,8 +1648,8 @@ static int enqueue_forward(GPT2 *g, DevModel *d, int M, int lm_from, bool distin
 
   const int F = d->F, ldq = d->qkv_ld;
   const int nqkv = qwen ? E + 2 * kv : 3 * E;
-  // batched decode of 16-32 tokens: o and down quantize inside their GEMMs
-  const bool fq = d->fuse_quant && i8 && g_use_mfma && !run && M >= kGemmMinM && M <= 32;
+  // batched decode of 5-32 tokens: o and down quantize inside their GEMMs
+  const bool fq = d->fuse_quant && i8 && g_use_mfma && !run && M >= kGemmMinMI8 && M <= 32;
   // a decode of up to 4 tokens: each layer's o, MLP and the next layer's
   // q|k|v in one launch (decode_tail.hip)
   const bool tail = !step && use_tail(d, M, run, distinct);
