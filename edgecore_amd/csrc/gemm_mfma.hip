@@ -145,16 +145,17 @@ constexpr size_t gemm_lds_bytes() {
 constexpr int kGmMaxTiles = 1024;         // tiles of a split launch
 constexpr int kGmPartInts = 1024 * 1024;  // 32-bit partial tiles of a split launch
 __device__ int gm_part[kGmPartInts];
+__device__ __attribute__((aligned(16))) int8_t gm_zero[16];  // the chunks past a row's end (never written)
 __device__ unsigned gm_cnt[kGmMaxTiles];
 
 // A: [M * NP][lda] elements (row m's part p at row m * NP + p), as: per-row
 // scale (int8 quantization scale, or the split's 2^e; 1 for bf16)
-// RAG: rows that may end inside a 16-byte chunk, operands at any address, the
-// check for values that are not finite (a form of its own: the others ran 1-2%
-// slower with its branches in them)
-template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool RAG = false>
+// DL: rows of whole aligned chunks, straight to LDS; without it, rows that may
+// end inside a 16-byte chunk and operands at any address, through registers,
+// with the check for values that are not finite.  PART: the row ends inside the
+// last stage (a form of its own: the test per stage cost whole stages 3-10%)
+template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool PART = false>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
-  static_assert(!(RAG && DL), "the direct-to-LDS form takes whole aligned stages");
   using Op = MfmaOp<OP>;
   using Acc = typename Op::Acc;
   constexpr int NP = Op::NP;
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   float e_old[RES ? TI : 1][RES ? JO : 1][4];
   {
     // N*K >= 4N bytes: valid for every column index (weights at odd addresses: the output's row 0)
-    const float *stand = RAG && ((uintptr_t)a.W & 3) ? a.out : (const float *)a.W;
+    const float *stand = !DL && ((uintptr_t)a.W & 3) ? a.out : (const float *)a.W;
     const float *wsp = a.ws ? a.ws : stand, *bvp = a.bias ? a.bias : stand;
     const float *ws2p = (SWI && a.ws2) ? a.ws2 : stand;
 #pragma unroll
@@ -265,17 +266,13 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   auto load = [&](int k0) {
     kl = k0;
 #pragma unroll
-    for (int j = 0; j < ACH; j++) {
-      const int8_t *p = arow[j] + min(k0 + 16 * acol[j], KB - 16);
-      ra[j] = RAG ? ld16(p) : *reinterpret_cast<const v4i *>(p);
-    }
+    for (int j = 0; j < ACH; j++)
+      ra[j] = ld16(arow[j] + min(k0 + 16 * acol[j], KB - 16));
 #pragma unroll
-    for (int j = 0; j < BCH; j++) {
-      const int8_t *p = brow[j] + min(k0 + 16 * bcol[j], KB - 16);
-      rb[j] = RAG ? ld16(p) : *reinterpret_cast<const v4i *>(p);
-    }
+    for (int j = 0; j < BCH; j++)
+      rb[j] = ld16(brow[j] + min(k0 + 16 * bcol[j], KB - 16));
   };
-  const bool rag = RAG && (KB & 15);  // the row ends inside a chunk
+  const bool rag = KB & 15;  // the row ends inside a chunk
   auto store = [&](int buf) {
     const v4i z = {0, 0, 0, 0};
     if (rag) {
@@ -349,9 +346,9 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     // no padding; chunk c of row r sits at chunk c ^ (r & 7) of the row, so
     // that the 16-byte fragment reads of 8 consecutive rows hit distinct
     // banks.  A wave instruction fills 8 rows: lane l takes row 8 u + l / 8
-    // and stores the row's chunk (l & 7) ^ (l / 8) at position l & 7.  Rows
-    // are K-complete (the launcher takes this path when K bytes are a
-    // multiple of kBK), so no chunk is past the row.
+    // and stores the row's chunk (l & 7) ^ (l / 8) at position l & 7.  In a
+    // last stage that the row ends in, lanes past its end load zeros instead
+    // (gm_zero; rows are whole 16-byte chunks).
     constexpr int RT = NP * BM + kBN;  // tile rows per stage
     constexpr int UPW = RT / 32;       // 8-row load instructions per wave and stage
     static_assert(RT % 32 == 0, "tile rows");
@@ -378,9 +375,17 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     }
     auto dload = [&](int k0, int buf) {
       int8_t *base = lds + (size_t)buf * RT * kBK + (size_t)wave * UPW * 8 * kBK;
+      if (!PART || k0 + kBK <= KB) {  // uniform
 #pragma unroll
-      for (int u = 0; u < UPW; u++)
-        __builtin_amdgcn_global_load_lds((gvoid *)(src[u] + k0), (lvoid *)(base + u * 8 * kBK), 16, 0, 0);
+        for (int u = 0; u < UPW; u++)
+          __builtin_amdgcn_global_load_lds((gvoid *)(src[u] + k0), (lvoid *)(base + u * 8 * kBK), 16, 0, 0);
+      } else {
+        const bool in = k0 + 16 * lchk < KB;
+#pragma unroll
+        for (int u = 0; u < UPW; u++)
+          __builtin_amdgcn_global_load_lds((gvoid *)(in ? src[u] + k0 : gm_zero), (lvoid *)(base + u * 8 * kBK), 16, 0,
+                                           0);
+      }
     };
     const int sw = lr & 7;  // fragment rows are 16-aligned: row & 7 == lr & 7
     // NB stage buffers, NB - 1 stages in flight: stage s is waited for (each
@@ -490,7 +495,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     if (t == 0) __hip_atomic_store(&gm_cnt[tl], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  if constexpr (!I8 && RAG) {
+  if constexpr (!I8 && !DL) {
     if (a.Af) {  // uniform
       bool bad = false;
 #pragma unroll
@@ -583,9 +588,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-#ifndef EC_GEMM_DL
-#define EC_GEMM_DL 1
-#endif
 // K splits of a launch of T tiles over ns K stages: none when the tiles
 // already fill the CUs or the rows are short (under 16 stages: C2's q|k|v,
 // o and fc at 12 stages ran 8.6 -> 11.9, 8.6 -> 10.3 and 14.6 -> 18.7 us
@@ -609,17 +611,19 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   // split K for few tiles over long rows: C2's 128-token down projection
   // (24 tiles of 32 x 128 over 48 stages of K) ran each tile's whole K on
   // one CU while 232 CUs idled
-  const bool dl = EC_GEMM_DL && (a.K * MfmaOp<OP>::EB) % kBK == 0 && (a.lda * MfmaOp<OP>::EB) % kBK == 0 &&
-                  aligned16(a.A) && aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2)) && !a.Af;
-  const bool rag = a.Af || (a.K * MfmaOp<OP>::EB) % 16 || (a.lda * MfmaOp<OP>::EB) % 16 || !aligned16(a.A) ||
-                   !aligned16(a.W) || (EPI == EPI_SWIGLU && !aligned16(a.W2));
+  // rows of whole aligned 16-byte chunks go straight to LDS, any others through
+  // registers.  (Rows that were no whole number of 128-byte stages did too: 64
+  // x 4856 x 896 bf16 67.9 us, 23.0 so; 120 x 8944 x 1536 int8 37.3 and 18.0.)
+  const bool dl = (a.K * MfmaOp<OP>::EB) % 16 == 0 && (a.lda * MfmaOp<OP>::EB) % 16 == 0 && aligned16(a.A) &&
+                  aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2)) && !a.Af;
   const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM) : 1;
   const dim3 grid(8 * ((T + 7) / 8), ks);
+  const bool part = (a.K * MfmaOp<OP>::EB) % kBK != 0;
   if constexpr (BM == 32) {
     static_assert(gemm_lds_bytes<OP, 32, true, 4>() <= 158 * 1024, "split K: 4 stage buffers per CU");
     if (ks > 1) {
-      klaunch((gemm_mfma_kernel<OP, 32, EPI, true, 4, true>), grid, dim3(256), gemm_lds_bytes<OP, 32, true, 4>(), s,
-              a);
+      klaunch(part ? gemm_mfma_kernel<OP, 32, EPI, true, 4, true, true> : gemm_mfma_kernel<OP, 32, EPI, true, 4, true>,
+              grid, dim3(256), gemm_lds_bytes<OP, 32, true, 4>(), s, a);
       return hipGetLastError();
     }
   }
@@ -631,16 +635,17 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   const int bpc = T * ks <= 256 ? 1 : 2;
   const size_t budget = (size_t)(158 * 1024) / bpc;
   constexpr size_t l4 = gemm_lds_bytes<OP, BM, true, 4>(), l3 = gemm_lds_bytes<OP, BM, true, 3>();
+  // (a buffer count that never fits is not instantiated)
+  constexpr int n4 = l4 <= 158 * 1024 ? 4 : 2, n3 = l3 <= 158 * 1024 ? 3 : 2;
   if (dl && T <= 512 && l4 <= budget)
-    klaunch((gemm_mfma_kernel<OP, BM, EPI, true, l4 <= 158 * 1024 ? 4 : 2>), grid, dim3(256),
-            gemm_lds_bytes<OP, BM, true, l4 <= 158 * 1024 ? 4 : 2>(), s, a);
+    klaunch(part ? gemm_mfma_kernel<OP, BM, EPI, true, n4, false, true> : gemm_mfma_kernel<OP, BM, EPI, true, n4>, grid,
+            dim3(256), gemm_lds_bytes<OP, BM, true, n4>(), s, a);
   else if (dl && T <= 512 && l3 <= budget)
-    klaunch((gemm_mfma_kernel<OP, BM, EPI, true, l3 <= 158 * 1024 ? 3 : 2>), grid, dim3(256),
-            gemm_lds_bytes<OP, BM, true, l3 <= 158 * 1024 ? 3 : 2>(), s, a);
-  else if (dl) klaunch((gemm_mfma_kernel<OP, BM, EPI, true>), grid, dim3(256), gemm_lds_bytes<OP, BM, true>(), s, a);
-  else if (rag)
-    klaunch((gemm_mfma_kernel<OP, BM, EPI, false, 2, false, true>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s,
-            a);
+    klaunch(part ? gemm_mfma_kernel<OP, BM, EPI, true, n3, false, true> : gemm_mfma_kernel<OP, BM, EPI, true, n3>, grid,
+            dim3(256), gemm_lds_bytes<OP, BM, true, n3>(), s, a);
+  else if (dl)
+    klaunch(part ? gemm_mfma_kernel<OP, BM, EPI, true, 2, false, true> : gemm_mfma_kernel<OP, BM, EPI, true>, grid,
+            dim3(256), gemm_lds_bytes<OP, BM, true>(), s, a);
   else klaunch((gemm_mfma_kernel<OP, BM, EPI, false>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s, a);
   return hipGetLastError();
 }
@@ -711,12 +716,13 @@ __device__ __forceinline__ float split_max(float mx, float x) {
 // the others zero.
 __device__ __forceinline__ int split_exp(float mx) { return mx > 0.0f ? max(ilogbf(mx) - 14, -100) : 0; }
 
-// one block of 256 threads per row: the row's 16-bit parts and scale.  VEC:
-// rows of whole aligned 8-element chunks, read and written 16 bytes at a time
+// one block of 256 threads per row: the row's 16-bit parts and scale.  VEC (4
+// or 8, 0 for any row): rows of whole aligned VEC-element chunks, read and written
+// in one piece, four elements where eight would leave threads of the block idle
 // (one element at a time, 300 x 3072 x 768 fp16 took 25.9 us with the GEMM, 22.3 so),
 // up to kSplitStrips of them per thread kept between the maximum and the parts.
 constexpr int kSplitStrips = 2;
-template <int OP, bool VEC>
+template <int OP, int VEC>
 __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int K, uint16_t *out, int ldo,
                                                     float *rs) {
   constexpr int NP = MfmaOp<OP>::NP;
@@ -725,15 +731,19 @@ __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int
   const float *row = x + (size_t)m * ldx;
   uint16_t *o = out + (size_t)m * NP * ldo;
   int e = 0;
-  if constexpr (VEC) {
+  if constexpr (VEC > 0) {
     auto chunk = [&](int c, float *f) {
-      const float4 a = *reinterpret_cast<const float4 *>(row + 8 * c), b = *reinterpret_cast<const float4 *>(row + 8 * c + 4);
-      f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w, f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
-    };
-    auto parts = [&](int c, const float *f) {
-      v4u w[NP];
 #pragma unroll
-      for (int i = 0; i < 8; i += 2) {
+      for (int i = 0; i < VEC; i += 4) {
+        const float4 a = *reinterpret_cast<const float4 *>(row + VEC * c + i);
+        f[i] = a.x, f[i + 1] = a.y, f[i + 2] = a.z, f[i + 3] = a.w;
+      }
+    };
+    typedef uint32_t vec_t __attribute__((ext_vector_type(VEC / 2)));
+    auto parts = [&](int c, const float *f) {
+      vec_t w[NP];
+#pragma unroll
+      for (int i = 0; i < VEC; i += 2) {
         uint16_t a[NP], b[NP];
         split_parts<OP>(f[i], e, a);
         split_parts<OP>(f[i + 1], e, b);
@@ -741,10 +751,10 @@ __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int
         for (int p = 0; p < NP; p++) w[p][i / 2] = a[p] | ((uint32_t)b[p] << 16);
       }
 #pragma unroll
-      for (int p = 0; p < NP; p++) *reinterpret_cast<v4u *>(o + (size_t)p * ldo + 8 * c) = w[p];
+      for (int p = 0; p < NP; p++) *reinterpret_cast<vec_t *>(o + (size_t)p * ldo + VEC * c) = w[p];
     };
-    const int nc = K / 8;
-    float f[kSplitStrips][8];
+    const int nc = K / VEC;
+    float f[kSplitStrips][VEC];
 #pragma unroll
     for (int s = 0; s < kSplitStrips; s++) chunk(min(t + 256 * s, nc - 1), f[s]);
     if constexpr (OP == OP_F16) {
@@ -752,12 +762,12 @@ __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int
 #pragma unroll
       for (int s = 0; s < kSplitStrips; s++)
 #pragma unroll
-        for (int i = 0; i < 8; i++) mx = split_max(mx, f[s][i]);
+        for (int i = 0; i < VEC; i++) mx = split_max(mx, f[s][i]);
       for (int c = t + 256 * kSplitStrips; c < nc; c += 256) {
-        float g[8];
+        float g[VEC];
         chunk(c, g);
 #pragma unroll
-        for (int i = 0; i < 8; i++) mx = split_max(mx, g[i]);
+        for (int i = 0; i < VEC; i++) mx = split_max(mx, g[i]);
       }
       e = split_exp(block_max256(mx, red));
     }
@@ -765,7 +775,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float *x, int ldx, int
     for (int s = 0; s < kSplitStrips; s++)
       if (t + 256 * s < nc) parts(t + 256 * s, f[s]);
     for (int c = t + 256 * kSplitStrips; c < nc; c += 256) {
-      float g[8];
+      float g[VEC];
       chunk(c, g);
       parts(c, g);
     }
@@ -1232,9 +1242,10 @@ hipError_t split_rows16(const GemvArgs &a, int wt, uint16_t *parts, int ldp, flo
   if ((wt != WT_F16 && wt != WT_BF16) || a.M < 1 || a.K < 1) return hipErrorInvalidValue;
   if (!parts || !rs || ldp < a.K || ldp % 8 || !aligned16(parts)) return hipErrorInvalidValue;
   const float *x = (const float *)a.A;
-  const bool vec = a.K % 8 == 0 && a.lda % 4 == 0 && aligned16(x);
-  auto k = wt == WT_F16 ? (vec ? split_kernel<OP_F16, true> : split_kernel<OP_F16, false>)
-                        : (vec ? split_kernel<OP_BF16, true> : split_kernel<OP_BF16, false>);
+  const int vec = a.K % 8 == 0 && a.lda % 4 == 0 && aligned16(x) ? (a.K <= 1024 ? 4 : 8) : 0;
+  auto k = wt == WT_F16
+               ? (vec == 8 ? split_kernel<OP_F16, 8> : vec == 4 ? split_kernel<OP_F16, 4> : split_kernel<OP_F16, 0>)
+               : (vec == 8 ? split_kernel<OP_BF16, 8> : vec == 4 ? split_kernel<OP_BF16, 4> : split_kernel<OP_BF16, 0>);
   klaunch(k, dim3(a.M), dim3(256), 0, s, x, a.lda, a.K, parts, ldp, rs);
   return hipGetLastError();
 }

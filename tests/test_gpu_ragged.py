@@ -105,3 +105,28 @@ def test_w16_not_finite(M, bf16):
     assert inf.any() and np.array_equal(got[inf], want[inf].astype(np.float32))
     mag = np.where(np.isfinite(A), np.abs(A), 0).astype(np.float64) @ np.where(np.isfinite(Bf), np.abs(Bf), 0).T
     assert np.all(np.abs(got[fin] - want[fin]) <= 2.0 * K * 2.0 ** -24 * mag[fin])
+
+
+# rows of whole 16-byte chunks that end inside a 128-byte stage of the tile
+# kernel: one chunk past and short of a stage, each row tile, split K (few
+# tiles, 16 or more stages), 2 to 4 stage buffers
+STAGE_SHAPES = [(33, 16, 40), (40, 112, 130), (40, 144, 130), (64, 2064, 200), (130, 4848, 129), (600, 1008, 9001)]
+
+
+@pytest.mark.parametrize("M,K,N", STAGE_SHAPES)
+def test_int8_partial_stage(M, K, N):
+    test_int8_bit_exact(M, K, N)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M,K,N", [(M, K // 2, N) for M, K, N in STAGE_SHAPES])
+def test_w16_partial_stage(M, K, N, bf16):
+    rng = np.random.default_rng(M + K + N)
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    B = (rng.normal(0, 0.02, (N, K)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) if bf16 else \
+        rng.normal(0, 0.02, (N, K)).astype(np.float16).view(np.uint16)
+    Bf = (B.astype(np.uint32) << 16).view(np.float32) if bf16 else B.view(np.float16).astype(np.float32)
+    got = (ec.gemm_bf16_fp32 if bf16 else ec.gemm_fp16_fp32)(A, B)
+    want = A.astype(np.float64) @ Bf.T.astype(np.float64)
+    bound = 2.0 * K * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(Bf.T).astype(np.float64)) + 1e-30
+    assert np.all(np.abs(got - want) <= bound)
