@@ -129,9 +129,9 @@ __device__ __forceinline__ float redo_dot(const GemvArgs &a, const void *W, int 
 
 // NB stage buffers (2, or up to 4 in the direct-to-LDS form); the
 // direct-to-LDS form (DL) has unpadded rows
-template <int OP, int BM, bool DL, int NB = 2>
+template <int OP, int BM, bool DL, int NB = 2, int BN = kBN>
 constexpr size_t gemm_lds_bytes() {
-  return (size_t)NB * (MfmaOp<OP>::NP * BM + kBN) * (DL ? kBK : kPitch);
+  return (size_t)NB * (MfmaOp<OP>::NP * BM + BN) * (DL ? kBK : kPitch);
 }
 
 // Split K of the tiled kernel: gridDim.y blocks share a tile, each taking a
@@ -154,7 +154,7 @@ __device__ unsigned gm_cnt[kGmMaxTiles];
 // end inside a 16-byte chunk and operands at any address, through registers,
 // with the check for values that are not finite.  PART: the row ends inside the
 // last stage (a form of its own: the test per stage cost whole stages 3-10%)
-template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool PART = false>
+template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool PART = false, int BN = kBN>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   using Op = MfmaOp<OP>;
   using Acc = typename Op::Acc;
@@ -163,17 +163,17 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   constexpr bool SWI = EPI == EPI_SWIGLU;
   constexpr bool RES = EPI == EPI_RESID || EPI == EPI_BIAS_RESID;
   constexpr bool GELU = EPI == EPI_GELU || EPI == EPI_BIAS_GELU;
-  constexpr int WM = BM / 2, WN = kBN / 2;   // wave tile
+  constexpr int WM = BM / 2, WN = BN / 2;   // wave tile
   constexpr int TI = WM / 16, TJ = WN / 16;  // 16 x 16 MFMA tiles per wave
   constexpr int CPR = kBK / 16;              // 16-byte chunks per tile row and stage
   constexpr int ACH = NP * BM * CPR / 256;   // A chunks per thread and stage
-  constexpr int BCH = kBN * CPR / 256;       // B chunks per thread and stage
-  constexpr int NOUT = SWI ? kBN / 2 : kBN;  // output columns per block
+  constexpr int BCH = BN * CPR / 256;       // B chunks per thread and stage
+  constexpr int NOUT = SWI ? BN / 2 : BN;  // output columns per block
   static_assert(ACH >= 1 && BCH >= 1 && TJ % 2 == 0 && NP * BM * CPR % 256 == 0, "tile shape");
 
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
   int8_t *la = lds;                            // [2][NP][BM][kPitch]
-  int8_t *lb = lds + 2 * NP * BM * kPitch;     // [2][kBN][kPitch]
+  int8_t *lb = lds + 2 * NP * BM * kPitch;     // [2][BN][kPitch]
   __shared__ uint64_t etab[SWI ? 32 : 1];
 
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   // clamped into the matrix and absent vectors read a stand-in (the weight
   // rows); the values are selected at use.
   constexpr int JO = SWI ? TJ / 2 : TJ;  // output column tiles
-  const int lrow0 = m0 + wm * WM + 4 * lq, lcol0 = n0 + (SWI ? wn * (kBN / 4) : wn * WN) + lr;
+  const int lrow0 = m0 + wm * WM + 4 * lq, lcol0 = n0 + (SWI ? wn * (BN / 4) : wn * WN) + lr;
   float e_as[TI][4], e_bs[JO], e_bv[JO], e_bs2[JO];
   float e_old[RES ? TI : 1][RES ? JO : 1][4];
   {
@@ -250,9 +250,9 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     bcol[j] = c % CPR;
     const int8_t *W = (const int8_t *)a.W;
     int n = n0 + r;
-    if (SWI && r >= kBN / 2) {
+    if (SWI && r >= BN / 2) {
       W = (const int8_t *)a.W2;
-      n = n0 + r - kBN / 2;
+      n = n0 + r - BN / 2;
     }
     brow[j] = W + (size_t)min(n, N - 1) * KB;
     boff[j] = r * kPitch + 16 * bcol[j];
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
       *reinterpret_cast<v4i *>(la + buf * NP * BM * kPitch + aoff[j]) = kl + 16 * acol[j] < KB ? ra[j] : z;
 #pragma unroll
     for (int j = 0; j < BCH; j++)
-      *reinterpret_cast<v4i *>(lb + buf * kBN * kPitch + boff[j]) = kl + 16 * bcol[j] < KB ? rb[j] : z;
+      *reinterpret_cast<v4i *>(lb + buf * BN * kPitch + boff[j]) = kl + 16 * bcol[j] < KB ? rb[j] : z;
   };
 
   // B tile rows of this wave's column tiles: plain, or gate (j < TJ/2) and up
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   for (int j = 0; j < TJ; j++) {
     if constexpr (SWI) {
       const int jj = j % (TJ / 2);
-      bt[j] = (j < TJ / 2 ? 0 : kBN / 2) + wn * (kBN / 4) + 16 * jj;
+      bt[j] = (j < TJ / 2 ? 0 : BN / 2) + wn * (BN / 4) + 16 * jj;
     } else {
       bt[j] = wn * WN + 16 * j;
     }
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
       const int buf = s & 1;
       if (s + 1 < ns) load(kb0 + (s + 1) * kBK);
       const int8_t *ta = la + buf * NP * BM * kPitch + (wm * WM + lr) * kPitch + 16 * lq;
-      const int8_t *tb = lb + buf * kBN * kPitch + lr * kPitch + 16 * lq;
+      const int8_t *tb = lb + buf * BN * kPitch + lr * kPitch + 16 * lq;
   #pragma unroll
       for (int kk = 0; kk < kBK / 64; kk++) {
         v4i fa[NP][TI], fb[TJ];
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     // and stores the row's chunk (l & 7) ^ (l / 8) at position l & 7.  In a
     // last stage that the row ends in, lanes past its end load zeros instead
     // (gm_zero; rows are whole 16-byte chunks).
-    constexpr int RT = NP * BM + kBN;  // tile rows per stage
+    constexpr int RT = NP * BM + BN;  // tile rows per stage
     constexpr int UPW = RT / 32;       // 8-row load instructions per wave and stage
     static_assert(RT % 32 == 0, "tile rows");
     typedef __attribute__((address_space(1))) const void gvoid;
@@ -366,9 +366,9 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
         const int rb = r - NP * BM;
         const int8_t *W = (const int8_t *)a.W;
         int n = n0 + rb;
-        if (SWI && rb >= kBN / 2) {
+        if (SWI && rb >= BN / 2) {
           W = (const int8_t *)a.W2;
-          n = n0 + rb - kBN / 2;
+          n = n0 + rb - BN / 2;
         }
         src[u] = W + (size_t)min(n, N - 1) * KB + 16 * lchk;
       }
@@ -604,6 +604,24 @@ int gemm_ksplit(int T, int ns, int BM) {
   return (ns + kper - 1) / kper;
 }
 
+// 32 x 64 tiles where 32 x 128 ones would be fewer than 128 blocks, which left
+// more than half of the CUs idle: twice the blocks, each with half the multiplies
+// and epilogue per stage.  128 x 768 x 3072 fp16 bias + GELU (96 tiles) 17.0 ->
+// 12.5 us, 100 x 896 x 896 bf16 (28) 13.2 -> 10.9, 100 x 1536 x 3000 int8 GELU
+// (96) 14.0 -> 9.4, 40 x 1536 x 4096 int8 (64) 8.1 -> 6.1.  Rows of 16 or more
+// stages split K first.
+constexpr int kNarrowTiles = 128;
+
+template <int OP, int EPI>
+hipError_t launch_narrow(const GemvArgs &a, bool part, hipStream_t s) {
+  constexpr int BN = 64, NOUT = EPI == EPI_SWIGLU ? BN / 2 : BN;
+  const int T = ((a.N + NOUT - 1) / NOUT) * ((a.M + 31) / 32);
+  klaunch(part ? gemm_mfma_kernel<OP, 32, EPI, true, 4, false, true, BN>
+               : gemm_mfma_kernel<OP, 32, EPI, true, 4, false, false, BN>,
+          dim3(8 * ((T + 7) / 8), 1), dim3(256), gemm_lds_bytes<OP, 32, true, 4, BN>(), s, a);
+  return hipGetLastError();
+}
+
 template <int OP, int BM, int EPI>
 hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   constexpr int NOUT = EPI == EPI_SWIGLU ? kBN / 2 : kBN;
@@ -626,6 +644,7 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
               grid, dim3(256), gemm_lds_bytes<OP, 32, true, 4>(), s, a);
       return hipGetLastError();
     }
+    if (dl && T < kNarrowTiles) return launch_narrow<OP, EPI>(a, part, s);
   }
   // grids of at most two tiles per CU: the most stage buffers (up to 4) with
   // which the tiles a CU holds at once still fit its LDS, so that 2-3
