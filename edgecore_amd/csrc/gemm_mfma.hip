@@ -671,12 +671,26 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
 
 template <int OP, int EPI>
 hipError_t launch_epi(const GemvArgs &a, int bm, hipStream_t s) {
-  // the largest row tile that still gives every CU a block or more, else the
-  // smallest (N = 896 at M = 2048: 448 blocks of 32 rows beat 224 of 64 rows,
-  // 9.7 against 10.7 us for K = 896 and 34.0 against 35.5 us for K = 4864)
+  // Row tiles by the number of blocks they give, K x N at M rows, us at 32 / 64
+  // / 128 rows.  int8 SwiGLU: 1536 x 8960 at 2048 140 / 92 / 85 (2240 blocks of
+  // 128), at 1024 61 / 45 / 45 (1120); 896 x 4864 at 777 21 / 18 / 23 (532),
+  // at 512 14 / 13 / 15, at 1500 30 at 128 (912) and 31 at 64; N = 896 at 2048 rows: 448 blocks of 32 beat 224 of 64
+  // (9.7 and 10.7, K = 4864 34.0 and 35.5).  The 16-bit parts double or triple
+  // the activation tile, so 128 rows leave one block per CU: fp16 896 x 4864
+  // SwiGLU at 777 44 / 40 / 64 (988 blocks of 64), at 512 30 / 33 / 45 (608),
+  // 1536 x 8960 at 2048 313 / 271 / 290, stores 1000 x 5000 at 640 38 / 32
+  // (400 of 64), GELU 768 x 3072 at 1024 36 / 40 (384); bf16 at 777 55 / 65 / 84, 1536 x 8960
+  // at 2048 410 / 446 / 383, 896 x 4864 at 2048 150 / 166 / 140 (1216 of 128);
+  // bf16 stores 896 x 9728 at 777 53 / 48 / 79, at 512 38 / 38 / 54.
   constexpr int NOUT = EPI == EPI_SWIGLU ? kBN / 2 : kBN;
-  const long gx = (a.N + NOUT - 1) / NOUT;
-  if (bm == 0) bm = gx * ((a.M + 127) / 128) >= 256 ? 128 : gx * ((a.M + 63) / 64) >= 256 ? 64 : 32;
+  const long gx = (a.N + NOUT - 1) / NOUT, t128 = gx * ((a.M + 127) / 128), t64 = gx * ((a.M + 63) / 64);
+  if (bm == 0) {
+    constexpr bool heavy = EPI == EPI_SWIGLU || EPI == EPI_GELU;  // epilogues worth spreading
+    if (OP == OP_I8) bm = t128 >= 768 ? 128 : t64 >= 256 ? 64 : 32;
+    else if (OP == OP_F16) bm = t64 >= (heavy ? 800 : 256) ? 64 : 32;
+    else if (EPI == EPI_SWIGLU) bm = t128 >= 1200 ? 128 : 32;
+    else bm = t64 >= 500 ? 64 : 32;
+  }
   if (bm == 128) return launch_bm<OP, 128, EPI>(a, s);
   if (bm == 64) return launch_bm<OP, 64, EPI>(a, s);
   return launch_bm<OP, 32, EPI>(a, s);
