@@ -387,7 +387,7 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
 // finite outside a token's range does not reach it.
 //
 // 2048 tokens, 14 heads of 64: 363 us with the scores in LDS and DPP products,
-// 252 us here; 12 heads of 128: 667 and 319 us; 500 tokens, 14 heads: 54 and
+// 251 (another card 266) here; 12 heads of 128: 667 and 317 us; 500 tokens, 14 heads: 55 and
 // 43 us.  The adds and products alone are about 125 us of that at 2.3 GHz, the
 // exponentials 25 us; the rest is the output phase's one wave per SIMD and
 // block (198 cycles per four positions where the SIMD could do 72).
