@@ -70,11 +70,6 @@ struct GemvArgs {
   // group] (np_out >= the number of column groups)
   float *pmax_out;
   int np_out;
-  // 16-bit matrix-core GEMM: when set, the fp32 rows behind the 16-bit parts
-  // (stride ldaf); an output that the parts make NaN is then summed again from
-  // them, so that weights that are not finite give what an fp32 sum gives
-  const float *Af;
-  int ldaf;
 };
 
 // Weight types
@@ -133,7 +128,6 @@ hipError_t gemm_i8_skinny_q(const GemvArgs &a, int epi, hipStream_t s);
 // W / W2.
 int w16_parts(int wt);
 bool gemm_w16_ok(const GemvArgs &a, int wt, int epi);
-bool gemm_w16_any_ok(const GemvArgs &a, int wt, int epi);  // any K from 8, any alignment
 hipError_t gemm_w16(const GemvArgs &a, int wt, int epi, uint16_t *parts, int ldp, float *rs, hipStream_t s);
 hipError_t gemm_w16_tile(const GemvArgs &a, int wt, int epi, int bm, uint16_t *parts, int ldp, float *rs,
                          hipStream_t s);
@@ -141,6 +135,11 @@ hipError_t gemm_w16_tile(const GemvArgs &a, int wt, int epi, int bm, uint16_t *p
 hipError_t split_rows16(const GemvArgs &a, int wt, uint16_t *parts, int ldp, float *rs, hipStream_t s);
 hipError_t gemm_w16_parts(const GemvArgs &a, int wt, int epi, int bm, const uint16_t *parts, int ldp,
                           const float *rs, hipStream_t s);
+// 16-bit weights and fp32 rows of any length from 8 elements at any address, in
+// fp32 throughout and without a workspace (gemm_f32.hip): every epilogue but
+// argmax candidates, no weight scales
+bool gemm_f32_ok(const GemvArgs &a, int wt, int epi);
+hipError_t gemm_f32(const GemvArgs &a, int wt, int epi, hipStream_t s);
 // grid-size cap of the grid-stride GEMV (set from the CU count at init)
 void gemv_set_max_blocks(int n);
 int gemv_max_blocks();

@@ -34,9 +34,10 @@
 // bytes apart, so the 16-byte fragment reads of 8 consecutive lanes (16 rows,
 // same k) fall on distinct banks.  The activation tile holds NP parts (1 for
 // int8, 2 for fp16, 3 for bf16), part-major.
-// Rows whose length is no multiple of 16 bytes (and operands at any address)
+// int8 rows whose length is no multiple of 16 (and operands at any address)
 // take the register-staged form with unaligned 16-byte loads, the chunk that a
-// row ends in loaded from the row's last 16 bytes and its other bytes zeroed:
+// row ends in loaded from the row's last 16 bytes and its other bytes zeroed
+// (16-bit weights: gemm_f32.hip):
 // 333 x 1000 x 777 int8 took 970 us in the one-thread-per-output kernel that
 // these shapes had, its byte loads serial.
 //
@@ -113,20 +114,6 @@ __device__ __forceinline__ v4i tail16(v4i v, int c, int KB) {
   return v;
 }
 
-// The fp32 dot of activation row m with weight row n in order, for an output
-// whose 16-bit parts gave NaN: a weight that is not finite times a part that is
-// zero, or infinities of both signs among the parts.  Only where the caller
-// gives the fp32 rows (a.Af).
-template <int OP>
-__device__ __forceinline__ float redo_dot(const GemvArgs &a, const void *W, int m, int n) {
-  const float *x = a.Af + (size_t)m * a.ldaf;
-  const uint16_t *w = reinterpret_cast<const uint16_t *>(W) + (size_t)n * a.K;
-  float s = 0.0f;
-#pragma unroll 1
-  for (int k = 0; k < a.K; k++) s = __builtin_fmaf(x[k], w2f<OP == OP_BF16>(w[k]), s);
-  return s;
-}
-
 // NB stage buffers (2, or up to 4 in the direct-to-LDS form); the
 // direct-to-LDS form (DL) has unpadded rows
 template <int OP, int BM, bool DL, int NB = 2, int BN = kBN>
@@ -150,9 +137,9 @@ __device__ unsigned gm_cnt[kGmMaxTiles];
 
 // A: [M * NP][lda] elements (row m's part p at row m * NP + p), as: per-row
 // scale (int8 quantization scale, or the split's 2^e; 1 for bf16)
-// DL: rows of whole aligned chunks, straight to LDS; without it, rows that may
-// end inside a 16-byte chunk and operands at any address, through registers,
-// with the check for values that are not finite.  PART: the row ends inside the
+// DL: rows of whole aligned chunks, straight to LDS; without it (int8), rows
+// that may end inside a 16-byte chunk and operands at any address, through
+// registers.  PART: the row ends inside the
 // last stage (a form of its own: the test per stage cost whole stages 3-10%)
 template <int OP, int BM, int EPI, bool DL, int NB = 2, bool SPLIT = false, bool PART = false, int BN = kBN>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
@@ -169,6 +156,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
   constexpr int ACH = NP * BM * CPR / 256;   // A chunks per thread and stage
   constexpr int BCH = BN * CPR / 256;       // B chunks per thread and stage
   constexpr int NOUT = SWI ? BN / 2 : BN;  // output columns per block
+  static_assert(DL || I8, "16-bit parts are whole aligned chunks");
   static_assert(ACH >= 1 && BCH >= 1 && TJ % 2 == 0 && NP * BM * CPR % 256 == 0, "tile shape");
 
   extern __shared__ __attribute__((aligned(16))) int8_t lds[];
@@ -495,37 +483,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
     if (t == 0) __hip_atomic_store(&gm_cnt[tl], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  if constexpr (!I8 && !DL) {
-    if (a.Af) {  // uniform
-      bool bad = false;
-#pragma unroll
-      for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int j = 0; j < TJ; j++) {
-          const v4f w = acc[i][j];
-          bad = bad || w[0] != w[0] || w[1] != w[1] || w[2] != w[2] || w[3] != w[3];
-        }
-      if (bad) {  // this thread's outputs one by one
-#pragma unroll 1
-        for (int q = 0; q < TI * JO * 4; q++) {
-          const int m = lrow0 + 16 * (q / (4 * JO)) + (q & 3), n = lcol0 + 16 * ((q >> 2) % JO);
-          if (m >= M || n >= N) continue;
-          float x = redo_dot<OP>(a, a.W, m, n);
-          float *o = a.out + (size_t)m * a.ldo + n;
-          if constexpr (SWI) {
-            x = silu(x, etab) * redo_dot<OP>(a, a.W2, m, n);
-          } else {
-            if (a.bias) x = x + a.bias[n];
-            if constexpr (RES) x = *o + x;
-            if constexpr (GELU) x = gelu_new(x);
-          }
-          *o = x;
-        }
-        return;
-      }
-    }
-  }
-
   // ---- epilogue: lane holds D[4*lq + r][lr] of each tile ----
   // Every value of a column tile is computed before any of its stores, so
   // that the 4*TI independent chains (SiLU's expf and division, GELU's tanh)
@@ -633,7 +590,7 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   // registers.  (Rows that were no whole number of 128-byte stages did too: 64
   // x 4856 x 896 bf16 67.9 us, 23.0 so; 120 x 8944 x 1536 int8 37.3 and 18.0.)
   const bool dl = (a.K * MfmaOp<OP>::EB) % 16 == 0 && (a.lda * MfmaOp<OP>::EB) % 16 == 0 && aligned16(a.A) &&
-                  aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2)) && !a.Af;
+                  aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2));
   const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM) : 1;
   const dim3 grid(8 * ((T + 7) / 8), ks);
   const bool part = (a.K * MfmaOp<OP>::EB) % kBK != 0;
@@ -665,7 +622,9 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   else if (dl)
     klaunch(part ? gemm_mfma_kernel<OP, BM, EPI, true, 2, false, true> : gemm_mfma_kernel<OP, BM, EPI, true>, grid,
             dim3(256), gemm_lds_bytes<OP, BM, true>(), s, a);
-  else klaunch((gemm_mfma_kernel<OP, BM, EPI, false>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s, a);
+  else if constexpr (OP == OP_I8)
+    klaunch((gemm_mfma_kernel<OP, BM, EPI, false>), grid, dim3(256), gemm_lds_bytes<OP, BM, false>(), s, a);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
@@ -868,8 +827,8 @@ __device__ unsigned sk_cnt[kSkMaxGroups];
 // with the row scale quant_scale(max |a|) of the row maximum given as partial
 // maxima (a.pmax, a.np); the codes are quant_rows' (the same scale and the
 // same per-element code), so the floats equal the unfused GEMM's.
-// RAG: rows may end inside a 16-byte chunk (a kernel of its own: the chunk's
-// mask spilled registers of the others)
+// RAG (int8 only): rows may end inside a 16-byte chunk (a kernel of its own: the
+// chunk's mask spilled registers of the others)
 template <int OP, int TI, int NJ, int EPI, bool QA = false, bool RAG = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
   using Op = MfmaOp<OP>;
@@ -881,6 +840,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
   constexpr bool GELU = EPI == EPI_GELU || EPI == EPI_BIAS_GELU;
   static_assert(!SWI || NJ == 1, "SwiGLU blocks take one tile of gate and up rows");
   static_assert(!QA || I8, "fused quantization of int8 activations");
+  static_assert(!RAG || I8, "16-bit parts are whole chunks");
   constexpr int NB = SWI ? 2 : NJ;  // B tiles: NJ tiles of 16 rows, or 16 gate + 16 up rows
   constexpr int FR = TI * NP * (QA ? 4 : 1) + NB;  // 16-byte loads per lane and step
   constexpr int U = (FR <= 3 ? 8 : FR <= 5 ? 4 : 2) / (RAG && FR <= 5 ? 2 : 1);  // K steps per wave in flight (within 128 VGPRs)
@@ -995,10 +955,6 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
           for (int i = 0; i < TI; i++)
 #pragma unroll
             for (int p = 0; p < NP; p++) fa[u][i][p] = tail16(fa[u][i][p], 64 * st + 16 * lq, KB);
-          if constexpr (!I8) {  // a weight that is not finite would make NaN of a zero activation
-#pragma unroll
-            for (int j = 0; j < NB; j++) fb[u][j] = tail16(fb[u][j], 64 * st + 16 * lq, KB);
-          }
         }
         if constexpr (QA) {
           // the codes of the fragment's 16 elements, packed four per word
@@ -1132,10 +1088,8 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(GemvArgs a) {
     }
   } else {
     v = sum[0] * as;
-    if (a.Af && v != v) v = redo_dot<OP>(a, a.W, m, n);
     if constexpr (SWI) {
-      float u = sum[1] * as;
-      if (a.Af && u != u) u = redo_dot<OP>(a, a.W2, m, n);
+      const float u = sum[1] * as;
       v = silu(v, etab) * u;
     } else if (a.bias) {
       v = v + a.bias[n];
@@ -1203,8 +1157,8 @@ hipError_t launch_skinny_nj(const GemvArgs &a, int wpb, int ksplit, hipStream_t 
 // 7.2-7.7 us measured); down (K = 8960) goes from 12.6 to 10.2 us.
 template <int OP, int TI, int EPI, bool QA = false>
 hipError_t launch_skinny(const GemvArgs &a, int wpb, hipStream_t s) {
-  if constexpr (!QA)
-    if (a.K * MfmaOp<OP>::EB % 16) return launch_skinny_nj<OP, TI, 1, EPI, false, true>(a, wpb, 1, s);
+  if constexpr (!QA && OP == OP_I8)
+    if (a.K % 16) return launch_skinny_nj<OP, TI, 1, EPI, false, true>(a, wpb, 1, s);
   if constexpr (EPI != EPI_SWIGLU && TI == 1) {
     if (a.N >= 16 * 1024) return launch_skinny_nj<OP, TI, 4, EPI, QA>(a, wpb, 1, s);
     if (OP == OP_I8 && (a.N + 15) / 16 < 192 && (a.K + 63) / 64 >= 64) {
@@ -1258,11 +1212,6 @@ hipError_t gemm_i8(const GemvArgs &a, int epi, hipStream_t s) { return gemm_i8_t
 
 int w16_parts(int wt) { return wt == WT_BF16 ? 3 : 2; }
 
-bool gemm_w16_any_ok(const GemvArgs &a, int wt, int epi) {
-  return (wt == WT_F16 || wt == WT_BF16) && a.M >= 1 && a.N >= 1 && a.K >= 8 && a.lda >= a.K && a.A && a.W &&
-         !a.cand && !a.ws && !a.ws2 && (epi != EPI_SWIGLU || a.W2) && epi_ok(epi);
-}
-
 bool gemm_w16_ok(const GemvArgs &a, int wt, int epi) {
   if (wt != WT_F16 && wt != WT_BF16) return false;
   if (a.M < 1 || a.N < 1 || a.K < 8 || a.K % 8 || a.cand || a.ws || a.ws2) return false;
@@ -1285,7 +1234,7 @@ hipError_t split_rows16(const GemvArgs &a, int wt, uint16_t *parts, int ldp, flo
 
 hipError_t gemm_w16_parts(const GemvArgs &a, int wt, int epi, int bm, const uint16_t *parts, int ldp,
                           const float *rs, hipStream_t s) {
-  if (!gemm_w16_any_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
+  if (!gemm_w16_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
     return hipErrorInvalidValue;
   if (!parts || !rs || ldp < a.K || ldp % 8 || !aligned16(parts)) return hipErrorInvalidValue;
   GemvArgs q = a;
@@ -1308,7 +1257,7 @@ hipError_t gemm_w16_parts(const GemvArgs &a, int wt, int epi, int bm, const uint
 
 hipError_t gemm_w16_tile(const GemvArgs &a, int wt, int epi, int bm, uint16_t *parts, int ldp, float *rs,
                          hipStream_t s) {
-  if (!gemm_w16_any_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
+  if (!gemm_w16_ok(a, wt, epi) || (bm != 0 && bm != 16 && bm != 32 && bm != 64 && bm != 128))
     return hipErrorInvalidValue;
   hipError_t e = split_rows16(a, wt, parts, ldp, rs, s);
   if (e != hipSuccess) return e;

@@ -382,13 +382,14 @@ static hipError_t gemv_any(const GemvArgs &a, int wt, int epi, int pro, hipStrea
 // Rows that the vector kernels cannot read in aligned 16-byte loads (K no
 // multiple of 16, or of 8 with 16-bit weights; operands at other addresses) go
 // to the matrix cores, for any M: one thread per output with serial byte loads
-// (gemv_generic) took 970 us for 333 x 1000 x 777 int8, 8.5 us now.  Rows
-// shorter than 16 bytes stay there.
+// (gemv_generic) took 970 us for 333 x 1000 x 777 int8, 8.5 us now.  16-bit
+// weights in fp32 (gemm_f32), as there: the operands keep their bits and the
+// call needs no workspace.  Rows shorter than 16 bytes stay there.
 static bool unaligned_gemm_i8(const GemvArgs &a) {
   return g_use_mfma && !gemv_vector_ok(a, WT_I8, PRO_I8) && gemm_i8_any_ok(a, EPI_STORE);
 }
 static bool unaligned_gemm_w16(const GemvArgs &a, int wt) {
-  return g_use_mfma && !gemv_vector_ok(a, wt, PRO_F32) && gemm_w16_any_ok(a, wt, EPI_STORE);
+  return g_use_mfma && !gemv_vector_ok(a, wt, PRO_F32) && gemm_f32_ok(a, wt, EPI_STORE);
 }
 
 extern "C" int ec_gemm_int8_dev(float *C, const int8_t *A, const float *a_scale, const int8_t *B,
@@ -466,18 +467,6 @@ static int w16_workspace(int M, int ldp) {
   return 0;
 }
 
-// the same for calls that can do without: false where the workspace would have
-// to grow inside a stream capture, or cannot
-static bool w16_workspace_ready(int M, int ldp) {
-  if ((size_t)M * 3 * ldp <= g_w16_halves && (size_t)M <= g_w16_rows) return true;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(g_stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return false;
-  if (w16_workspace(M, ldp) == 0) return true;
-  (void)hipGetLastError();
-  g_err[0] = 0;
-  return false;
-}
-
 static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int K, int N, bool bf16) {
   EC_INIT();
   if (M < 0 || N < 0 || K < 0) return set_err(-1, "gemm: negative shape M=%d K=%d N=%d", M, K, N);
@@ -493,11 +482,8 @@ static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int 
     EC_LAUNCH("gemm_w16", bytes, gemm_w16(a, wt, EPI_STORE, g_w16_parts, ldp, g_w16_rs, g_stream));
     return 0;
   }
-  if (unaligned_gemm_w16(a, wt) && w16_workspace_ready(M, (K + 7) & ~7)) {
-    const int ldp = (K + 7) & ~7;
-    a.Af = A;
-    a.ldaf = K;
-    EC_LAUNCH("gemm_w16", bytes, gemm_w16(a, wt, EPI_STORE, g_w16_parts, ldp, g_w16_rs, g_stream));
+  if (unaligned_gemm_w16(a, wt)) {
+    EC_LAUNCH("gemm_f32", bytes, gemm_f32(a, wt, EPI_STORE, g_stream));
     return 0;
   }
   if (gemv_regs_faster(a, wt)) {
@@ -1452,12 +1438,8 @@ static int linear(GPT2 *g, DevModel *d, const char *fam, GemvArgs a, int wt, int
     EC_LAUNCH(gemm_family(fam), bytes, a.M <= 32 ? gemm_i8_skinny(a, epi, 0, s) : gemm_i8(a, epi, s));
     return 0;
   }
-  if (wt != WT_I8 && g_use_mfma && a.M <= d->ah_rows && a.K <= d->ah_ld && gemm_w16_any_ok(a, wt, epi)) {
-    a.Af = (const float *)a.A;
-    a.ldaf = a.lda;
-    EC_LAUNCH("split16", 4.0 * a.M * a.K * (1.0 + w16_parts(wt) / 2.0),
-              split_rows16(a, wt, d->ah, d->ah_ld, d->ahs, s));
-    EC_LAUNCH(gemm_family(fam), bytes, gemm_w16_parts(a, wt, epi, 0, d->ah, d->ah_ld, d->ahs, s));
+  if (wt != WT_I8 && g_use_mfma && gemm_f32_ok(a, wt, epi)) {
+    EC_LAUNCH(gemm_family(fam), bytes, gemm_f32(a, wt, epi, s));
     return 0;
   }
   EC_LAUNCH(fam, bytes, gemv_generic(a, wt, epi, s));

@@ -1,8 +1,9 @@
 """GEMMs whose rows are no whole number of 16-byte chunks, or whose operands lie
 at any address: the matrix-core kernels' unaligned loads and the mask of the
 chunk that a row ends in, against the oracle (int8: bit for bit; 16-bit: the
-fp32 bound of tests/test_gpu_kernels.py), and, for values that are not finite,
-the class (finite, which infinity, NaN) of an fp32 sum."""
+fp32 bound of tests/test_gpu_kernels.py, also for rows whose values are far
+apart or tiny), and, for values that are not finite, the class (finite, which
+infinity, NaN) of an fp32 sum."""
 import numpy as np
 import pytest
 
@@ -68,7 +69,12 @@ def _bits(x, bf16):
     return ((u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
 
 
-@pytest.mark.parametrize("M,K,N", SHAPES[:-1])
+# 16-bit: up to 16 and 32 rows without stages, above and for wide outputs the
+# tiles; one, two, three and more stages of 64
+W16_SHAPES = SHAPES[:-1] + [(5, 8, 3), (3, 17, 16400), (32, 129, 16385), (33, 63, 65), (70, 193, 200)]
+
+
+@pytest.mark.parametrize("M,K,N", W16_SHAPES)
 @pytest.mark.parametrize("bf16", [False, True])
 def test_w16_within_bound(M, K, N, bf16):
     rng = np.random.default_rng(M + K + N + bf16)
@@ -79,6 +85,76 @@ def test_w16_within_bound(M, K, N, bf16):
     want = A.astype(np.float64) @ Bf.astype(np.float64).T
     bound = 2.0 * K * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(Bf).astype(np.float64).T)
     assert np.all(np.abs(got - want) <= bound)
+
+
+def _in_order(A, Bf):
+    """The fp32 FMA sum over k in order (a product of 24 and at most 11 bits is
+    exact in float64)."""
+    s = np.zeros((A.shape[0], Bf.shape[0]), np.float32)
+    for k in range(A.shape[1]):
+        s = (A[:, k, None].astype(np.float64) * Bf[None, :, k].astype(np.float64) + s).astype(np.float32)
+    return s
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M", [5, 20, 64])
+@pytest.mark.parametrize("K", [9, 17, 33, 101, 1001])
+@pytest.mark.parametrize("rows", ["normal", 1e8, 1e10, 1e-36, 1e-40])
+def test_w16_activations_keep_their_bits(M, K, rows, bf16):
+    """Rows with one value 1e8 or 1e10 times the others (it meets zero weights,
+    so the others make the result) and rows down to subnormal values: the fp32
+    bound, 2^-149 per product for what underflows, and an error against 64 bits
+    that is no larger than that of the fp32 sum in order (5%: the two round
+    differently)."""
+    N = 200
+    rng = np.random.default_rng(K + M)
+    A, W = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 0.02, (N, K)).astype(np.float32)
+    if rows in (1e8, 1e10):
+        A[:, 2], W[:, 2] = rows, 0.0
+    elif rows != "normal":
+        A, W = (A * np.float64(rows)).astype(np.float32), W * 50
+    B = _bits(W, bf16)
+    Bf = (B.astype(np.uint32) << 16).view(np.float32) if bf16 else B.view(np.float16).astype(np.float32)
+    got = (ec.gemm_bf16_fp32 if bf16 else ec.gemm_fp16_fp32)(A, B)
+    want = A.astype(np.float64) @ Bf.astype(np.float64).T
+    mag = np.abs(A).astype(np.float64) @ np.abs(Bf).astype(np.float64).T
+    assert np.all(np.abs(got - want) <= 2.0 * K * 2.0 ** -24 * mag + K * 2.0 ** -149)
+    assert np.linalg.norm(got - want) <= 1.05 * np.linalg.norm(_in_order(A, Bf) - want)
+
+
+@pytest.mark.parametrize("off", [2, 6, 8])
+@pytest.mark.parametrize("M,K,N", [(3, 96, 40), (20, 128, 130), (40, 128, 130), (40, 100, 33)])
+def test_w16_any_address(M, K, N, off):
+    """Weights and activations that start anywhere (multiples of their size)."""
+    rng = np.random.default_rng(M + K + N + off)
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    B = rng.normal(0, 0.02, (N, K)).astype(np.float16)
+    oa = 4 * (off // 4)
+    bufs = [_at(A, oa), _at(B.view(np.uint16), off)]
+    try:
+        got = _dev(ec.lib().ec_gemm_fp16_fp32_dev, (M, N), bufs[0].ptr + oa, bufs[1].ptr + off, M, K, N)
+    finally:
+        for b in bufs:
+            b.close()
+    want = A.astype(np.float64) @ B.astype(np.float64).T
+    assert np.all(np.abs(got - want) <= 2.0 * K * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64).T))
+
+
+@pytest.mark.parametrize("precision", ["fp16", "bf16"])
+@pytest.mark.parametrize("shape", [dict(arch="gpt2", embd=36, heads=2, ffn=147), dict(arch="qwen2", embd=36, heads=2, kv_heads=1, ffn=147)],
+                         ids=["gpt2", "qwen2"])
+def test_forward_of_ragged_widths(tmp_path, shape, precision):
+    """Models whose every linear is ragged: each epilogue (bias, residual, GELU,
+    SwiGLU) at 1, 5, 20 and 70 rows against the oracle's logits."""
+    path = tmp_path / "m.ecm"
+    ec.synth(path, layers=2, ctx=128, vocab=300, precision=precision, seed=3, **shape)
+    om = oracle.OracleModel(path, 1, 128)
+    with ec.Model(path, 1, 128) as m:
+        for n in (1, 5, 20, 70):
+            toks, pos, sl = np.arange(n) * 7 % 300, np.arange(n), np.zeros(n, np.int32)
+            got, _ = m.forward(toks, pos, sl)
+            assert np.abs(got - om.forward(toks, pos, sl)).max() <= 1e-4
+    om.close()
 
 
 @pytest.mark.parametrize("M", [5, 40])
