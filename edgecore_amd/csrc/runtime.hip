@@ -441,30 +441,55 @@ extern "C" int ec_gemm_int8_epi_dev(int epi, int bm, float *C, const int8_t *A, 
   return 0;
 }
 
-// 16-bit parts of the kernel-ABI 16-bit GEMMs' activation rows, grown on demand
-static uint16_t *g_w16_parts = nullptr;
-static float *g_w16_rs = nullptr;
-static size_t g_w16_halves = 0, g_w16_rows = 0;
+// 16-bit parts of the kernel-ABI 16-bit GEMMs' activation rows, grown on demand.
+// A call captured on ec_stream() records a buffer's address in the caller's
+// graph, which may be replayed at any time: a buffer that a capture has seen is
+// not freed before ec_release.  A larger call retires it and takes twice its
+// size or more, so that all retired ones together are no larger than the one in
+// use (where the device has that much; else what the call needs).
+struct W16Buf {
+  void *p = nullptr;
+  size_t n = 0;           // bytes
+  bool recorded = false;  // a capture has seen p
+  void *retired[64] = {};
+  int nretired = 0;
+};
+static W16Buf g_w16_parts, g_w16_rs;
+
+static int w16_grow(W16Buf &b, size_t bytes, bool capturing) {
+  if (bytes > b.n) {
+    if (capturing)
+      return set_err(-3, "gemm: the workspace would grow inside a stream capture (run such a call before it)");
+    size_t want = bytes;
+    if (b.recorded) {
+      if (b.nretired == 64) return set_err(-3, "gemm: 64 workspaces are held for captured graphs");
+      b.retired[b.nretired++] = b.p;
+      want = bytes > 2 * b.n ? bytes : 2 * b.n;
+    } else if (b.p) {
+      EC_HIP(hipStreamSynchronize(g_stream));
+      EC_HIP(hipFree(b.p));
+    }
+    b.p = nullptr;
+    b.n = 0;
+    b.recorded = false;
+    if (want > bytes && dev_malloc(&b.p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      b.p = nullptr;
+      want = bytes;
+    }
+    if (!b.p) EC_HIP(dev_malloc(&b.p, want));
+    b.n = want;
+  }
+  b.recorded = b.recorded || capturing;
+  return 0;
+}
 
 static int w16_workspace(int M, int ldp) {
-  const size_t halves = (size_t)M * 3 * ldp;
-  if (halves > g_w16_halves) {
-    EC_HIP(hipStreamSynchronize(g_stream));
-    if (g_w16_parts) EC_HIP(hipFree(g_w16_parts));
-    g_w16_parts = nullptr;
-    g_w16_halves = 0;
-    EC_HIP(dev_malloc(&g_w16_parts, halves * sizeof(uint16_t)));
-    g_w16_halves = halves;
-  }
-  if ((size_t)M > g_w16_rows) {
-    EC_HIP(hipStreamSynchronize(g_stream));
-    if (g_w16_rs) EC_HIP(hipFree(g_w16_rs));
-    g_w16_rs = nullptr;
-    g_w16_rows = 0;
-    EC_HIP(dev_malloc(&g_w16_rs, (size_t)M * sizeof(float)));
-    g_w16_rows = M;
-  }
-  return 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  EC_HIP(hipStreamIsCapturing(g_stream, &cap));
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  const int r = w16_grow(g_w16_parts, (size_t)M * 3 * ldp * sizeof(uint16_t), capturing);
+  return r ? r : w16_grow(g_w16_rs, (size_t)M * sizeof(float), capturing);
 }
 
 static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int K, int N, bool bf16) {
@@ -479,7 +504,8 @@ static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int 
     const int ldp = (K + 7) & ~7;
     int r;
     if ((r = w16_workspace(M, ldp))) return r;
-    EC_LAUNCH("gemm_w16", bytes, gemm_w16(a, wt, EPI_STORE, g_w16_parts, ldp, g_w16_rs, g_stream));
+    EC_LAUNCH("gemm_w16", bytes,
+              gemm_w16(a, wt, EPI_STORE, (uint16_t *)g_w16_parts.p, ldp, (float *)g_w16_rs.p, g_stream));
     return 0;
   }
   if (unaligned_gemm_w16(a, wt)) {
@@ -514,7 +540,8 @@ extern "C" int ec_gemm_w16_epi_dev(int wt, int epi, int bm, float *C, const floa
   const int ldp = (K + 7) & ~7;
   int r;
   if ((r = w16_workspace(M, ldp))) return r;
-  EC_LAUNCH("gemm_w16", 0.0, gemm_w16_tile(a, wt, epi, bm, g_w16_parts, ldp, g_w16_rs, g_stream));
+  EC_LAUNCH("gemm_w16", 0.0,
+            gemm_w16_tile(a, wt, epi, bm, (uint16_t *)g_w16_parts.p, ldp, (float *)g_w16_rs.p, g_stream));
   return 0;
 }
 
@@ -2364,11 +2391,11 @@ extern "C" int ec_release(void) {
     if (g_kept_host.p) EC_HIP(hipHostFree(g_kept_host.p));
     g_kept_dev = g_kept_host = Staging{};
   }
-  if (g_w16_parts) EC_HIP(hipFree(g_w16_parts));
-  if (g_w16_rs) EC_HIP(hipFree(g_w16_rs));
-  g_w16_parts = nullptr;
-  g_w16_rs = nullptr;
-  g_w16_halves = g_w16_rows = 0;
+  for (W16Buf *b : {&g_w16_parts, &g_w16_rs}) {
+    if (b->p) EC_HIP(hipFree(b->p));
+    for (int i = 0; i < b->nretired; i++) EC_HIP(hipFree(b->retired[i]));
+    *b = W16Buf{};
+  }
   for (hipEvent_t &ev : g_touch_ev) {
     if (ev) EC_HIP(hipEventDestroy(ev));
     ev = nullptr;
