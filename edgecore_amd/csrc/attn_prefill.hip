@@ -707,12 +707,12 @@ __global__ __launch_bounds__(kMmWaves * 64, NT > 4 ? 2 : 4) void attn_prefill_mm
   }
 }
 
-// positions that one block of 16 tokens reads
-int mm_span(const AttnArgs &a) {
-  int r = a.max_npos;
-  if (a.window > 0 && a.window + kMmTok - 1 < r) r = a.window + kMmTok - 1;
-  return r;
+// positions that a block of qb consecutive tokens reads (any window up to
+// INT_MAX: no sum with it before the comparison)
+int pf_span(const AttnArgs &a, int qb) {
+  return a.window > 0 && a.window < a.max_npos - (qb - 1) ? a.window + qb - 1 : a.max_npos;
 }
+int mm_span(const AttnArgs &a) { return pf_span(a, kMmTok); }
 // the most positions whose scores the kernel's registers hold
 constexpr int kMmMaxSpan = 8 * kMmWaves * kPfTile;
 
@@ -744,11 +744,7 @@ void launch_mm_any(const AttnArgs &a, hipStream_t st) {
 }
 
 // score slots per token: the positions one block reads, window-bounded
-int pf_nsc(const AttnArgs &a, int qb) {
-  int r = a.max_npos;
-  if (a.window > 0 && a.window + qb - 1 < r) r = a.window + qb - 1;
-  return (r + 3) & ~3;
-}
+int pf_nsc(const AttnArgs &a, int qb) { return (pf_span(a, qb) + 3) & ~3; }
 
 // tile with 4 spare rows, the score slots of qb tokens and 4 spare floats,
 // plus the static expf table (256 bytes)

@@ -145,3 +145,16 @@ def test_prefill_value_not_finite_outside_a_tokens_range(hd, H):
     want = oracle.attention_rows(q, kc, vc, pos, sl, H, KVH, window=window)
     assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
     _check(got, want, np.arange(window, M - 1))
+
+
+@pytest.mark.parametrize("path", [0, 1, 2])
+@pytest.mark.parametrize("window", [2 ** 31 - 1, 2 ** 31 - 8, 2 ** 30])
+def test_window_beyond_every_position(window, path):
+    """A window that reaches past every position, up to the largest int, is no
+    window (more than 512 positions: several score tiles per wave)."""
+    M, H, KVH, hd, p0 = 20, 2, 1, 64, 700
+    _, q, kc, vc = _case(window % 1000 + path, M, H, KVH, hd, p0 + M, 1)
+    pos, sl = p0 + np.arange(M), np.zeros(M)
+    got = ec.attention_dev(q, kc, vc, pos, sl, H, KVH, window=window, path=path)
+    assert np.array_equal(got, ec.attention_dev(q, kc, vc, pos, sl, H, KVH, window=0, path=path))
+    _check(got, oracle.attention_rows(q, kc, vc, pos, sl, H, KVH), np.arange(M))
