@@ -401,6 +401,12 @@ __device__ __forceinline__ v16f mm_bcast(float a, float b) {  // block ABID of a
   return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, v16f{0}, 2, ABID, 0);
 }
 
+// LDS accesses of the wave's other lanes before it come before those after it
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // the tile registers by a uniform index: a branch per tile (a move of 16
 // registers in the taken one)
 template <int NT>
@@ -499,8 +505,10 @@ __global__ __launch_bounds__(kMmWaves * 64, NT > 4 ? 2 : 4) void attn_prefill_mm
 #pragma unroll 1
     for (int e0 = 0; e0 < HD; e0 += KH) {
       // the tile's rows, whole 128-byte lines per instruction, through this
-      // wave's part of the LDS: a lane reads its position's row (no barrier:
-      // one wave's LDS operations are in order)
+      // wave's part of the LDS: a lane reads its position's row, which other
+      // lanes wrote (no block barrier: one wave's LDS operations are in order;
+      // wave_order keeps the compiler from moving them)
+      wave_order();  // the previous rows are read
       {
         v4u kr[CPR];
 #pragma unroll
@@ -514,6 +522,7 @@ __global__ __launch_bounds__(kMmWaves * 64, NT > 4 ? 2 : 4) void attn_prefill_mm
           *reinterpret_cast<v4u *>(wbuf + w * kMmWaveLds + r * (2 * KH) + 16 * (kchk ^ swz(r))) = kr[i];
         }
       }
+      wave_order();
       const float *qa = qt + e0 * T + lane;
       v4u kc = *reinterpret_cast<const v4u *>(kld + (0 ^ ksw));
       float aq = qa[0];
