@@ -731,23 +731,18 @@ void launch_mm(const AttnArgs &a, hipStream_t st) {
   klaunch((attn_prefill_mm_kernel<HD, NT>), dim3(a.H, ngroups), dim3(kMmWaves * 64), mm_lds_bytes<HD>(), st, a, ngroups);
 }
 
-// Whether the matrix-core kernel takes a prompt: its scores fit the registers,
-// and at head_dim 128, where the other kernel spreads a short prompt over twice
-// the blocks (8 tokens each), it has at least 192 blocks: 12 heads of 128,
-// 128 tokens (96 blocks) 30.2 us there, 34.2 us here; 256 tokens (192 blocks)
-// 38.5 and 38.1 us; 64 tokens after 1500 (48 blocks) 99.6 and 111.5 us.  At
-// head_dim 64 it is faster from 16 tokens (27.7 -> 27.1 us) on.
-bool mm_takes(const AttnArgs &a) {
-  if (mm_span(a) > kMmMaxSpan) return false;
-  return a.hd != 128 || (long)a.H * ((a.M + kMmTok - 1) / kMmTok) >= 192;
-}
-
 // by the longest span: the fewest score registers that hold it (up to 2048
-// positions two blocks share a CU, beyond that one)
+// positions two blocks share a CU, beyond that one).  The two-tile form spills
+// none at head_dim 32 and 64 (16 registers at 128), the four-tile one 105 (102):
+// 1024 tokens, us, with two and with four tiles: 16 heads of 32 72 and 95 (86
+// with the scores in LDS), 14 heads of 64 83 and 96, 12 of 128 107 and 114.  A
+// three-tile form spilled 214 and was slower than the four-tile one (1400
+// tokens, 14 heads of 64: 159 and 145).
 template <int HD>
 void launch_mm_any(const AttnArgs &a, hipStream_t st) {
   const int n = mm_span(a);
   if (n <= kMmWaves * kPfTile) launch_mm<HD, 1>(a, st);
+  else if (n <= 2 * kMmWaves * kPfTile) launch_mm<HD, 2>(a, st);
   else if (n <= 4 * kMmWaves * kPfTile) launch_mm<HD, 4>(a, st);
   else launch_mm<HD, 8>(a, st);
 }
@@ -768,6 +763,25 @@ int pf_pick(const AttnArgs &a, int max_lds) {
   for (int i = 0; i < 2; i++)
     if (pf_lds_bytes(a, kPfShapes[i]) <= (size_t)max_lds) return i;
   return -1;
+}
+
+// the 8-token blocks that the other kernel makes of a prompt
+long pf_blocks8(const AttnArgs &a) { return (long)a.H * ((a.M + 7) / 8); }
+
+// Whether the matrix-core kernel takes a prompt: its scores fit the registers,
+// and the other kernel's blocks, twice as many and each with half the tokens,
+// would be more than one per CU.  There and here, us: 14 heads of 64, 144 tokens
+// (252 of its blocks) 24.7 and 29.2 after none, 54.8 and 71.2 after 1000, 131
+// and 151 after 3500; 152 tokens (266) 25.0 and 29.5, 69.0 and 71.4, 237 and
+// 152; 16 heads of 32, 128 tokens (256) after 3500 118 and 133, 136 (272) 212
+// and 133.  At head_dim 128 from 192 of its own blocks: 12 heads, 128 tokens
+// (96) 30.2 and 34.2, 256 tokens (192) 38.5 and 38.1; 64 tokens after 1500 (48)
+// 99.6 and 111.5.
+constexpr int kCus = 256;
+bool mm_takes(const AttnArgs &a, int max_lds) {
+  if (mm_span(a) > kMmMaxSpan) return false;
+  if (a.hd == 128) return (long)a.H * ((a.M + kMmTok - 1) / kMmTok) >= 192;
+  return pf_pick(a, max_lds) != 0 || pf_blocks8(a) > kCus;
 }
 
 // grid (head, token group): consecutive block ids, which the dispatcher deals
@@ -792,12 +806,12 @@ void launch_hd(const AttnArgs &a, int shape, hipStream_t st) {
 bool attention_prefill_ok(const AttnArgs &a, int max_lds) {
   if (!(a.hd == 32 || a.hd == 64 || a.hd == 128) || !attn_vec(a.hd, a.kv) || a.fuse_kv || a.M < 1) return false;
   if (a.ldq % 4 || ((uintptr_t)a.q & 15u)) return false;  // q rows read as float4
-  return mm_takes(a) || pf_pick(a, max_lds) >= 0;
+  return mm_takes(a, max_lds) || pf_pick(a, max_lds) >= 0;
 }
 
 hipError_t attention_prefill(const AttnArgs &a, int max_lds, hipStream_t st) {
   if (!attention_prefill_ok(a, max_lds)) return hipErrorInvalidValue;
-  if (mm_takes(a)) {
+  if (mm_takes(a, max_lds)) {
     if (a.hd == 64) launch_mm_any<64>(a, st);
     else if (a.hd == 128) launch_mm_any<128>(a, st);
     else launch_mm_any<32>(a, st);

@@ -115,15 +115,23 @@ def test_attention_dev_rejects_bad_arguments():
         ec.attention_dev(q, kc, vc, [0, 1, 2, 3], [0, 0, 1, 0], H, KVH)          # slot outside the cache
 
 
-# the matrix-core prefill kernel: 16 tokens per block (1, 15, 17, 33 of them),
-# 64-position tiles, 1 (span 512), 4 (2048) and 8 (4096) of them per wave, and
-# past that the other kernel; head_dim 128 takes it from 192 blocks on
+# the two prefill kernels at the edges of the matrix-core one: 16 tokens per
+# block (1, 15, 17, 33 of them), 64-position tiles, 1 (span 512), 2 (1024), 4
+# (2048) and 8 (4096) of them per wave, and past that the other kernel, which
+# also takes what is at most 256 of its 8-token blocks (the rows of few heads);
+# head_dim 128 takes the matrix-core one from 192 blocks on
 @pytest.mark.parametrize("H,KVH,hd,M,p0,window", [
     (2, 1, 64, 1, 0, 0), (2, 1, 64, 15, 49, 0), (2, 2, 64, 17, 48, 0), (3, 1, 64, 33, 479, 0), (2, 1, 64, 33, 480, 0),
     (2, 1, 64, 20, 2028, 0), (2, 1, 64, 21, 2028, 0), (1, 1, 64, 16, 4080, 0), (1, 1, 64, 16, 4081, 0),
     (2, 1, 64, 40, 700, 1), (2, 1, 64, 70, 0, 497), (2, 1, 64, 70, 430, 498), (2, 1, 32, 33, 500, 0),
     (2, 2, 32, 17, 2100, 0), (96, 8, 128, 31, 0, 0), (96, 8, 128, 32, 490, 0), (96, 8, 128, 17, 1000, 300),
-    (96, 8, 128, 17, 2040, 0)])
+    (96, 8, 128, 17, 2040, 0),
+    (257, 1, 64, 1, 0, 0), (130, 2, 64, 15, 49, 0), (86, 2, 64, 17, 48, 0), (128, 2, 64, 16, 500, 0),
+    (130, 2, 64, 16, 500, 0), (54, 2, 64, 33, 479, 0), (54, 2, 64, 33, 480, 0), (86, 2, 64, 20, 1004, 0),
+    (86, 2, 64, 21, 1004, 0), (86, 2, 64, 20, 2028, 0), (86, 2, 64, 21, 2028, 0), (130, 1, 64, 16, 4080, 0),
+    (130, 1, 64, 16, 4081, 0), (54, 2, 64, 40, 700, 1), (30, 2, 64, 70, 0, 497), (30, 2, 64, 70, 430, 498),
+    (30, 2, 64, 70, 900, 1009), (30, 2, 64, 70, 900, 1010), (54, 2, 32, 33, 500, 0), (86, 2, 32, 17, 1000, 0),
+    (86, 2, 32, 17, 2100, 0), (96, 8, 128, 32, 700, 0), (96, 8, 128, 17, 3000, 0)])
 def test_prefill_matrix_core_edges(H, KVH, hd, M, p0, window):
     rng, q, kc, vc = _case(M + p0 + hd + window, M, H, KVH, hd, p0 + M, 2)
     pos, sl = p0 + np.arange(M), np.ones(M)
@@ -132,7 +140,7 @@ def test_prefill_matrix_core_edges(H, KVH, hd, M, p0, window):
     _check(got, want, np.arange(M))
 
 
-@pytest.mark.parametrize("hd,H", [(64, 2), (128, 96)])
+@pytest.mark.parametrize("hd,H", [(64, 2), (64, 60), (128, 96)])
 def test_prefill_value_not_finite_outside_a_tokens_range(hd, H):
     """An infinity in the last position's value reaches that position's token
     alone, and one before a window no token inside it."""
@@ -147,12 +155,12 @@ def test_prefill_value_not_finite_outside_a_tokens_range(hd, H):
     _check(got, want, np.arange(window, M - 1))
 
 
-@pytest.mark.parametrize("path", [0, 1, 2])
+@pytest.mark.parametrize("path,H", [(0, 2), (0, 88), (1, 2), (2, 2)])
 @pytest.mark.parametrize("window", [2 ** 31 - 1, 2 ** 31 - 8, 2 ** 30])
-def test_window_beyond_every_position(window, path):
+def test_window_beyond_every_position(window, path, H):
     """A window that reaches past every position, up to the largest int, is no
     window (more than 512 positions: several score tiles per wave)."""
-    M, H, KVH, hd, p0 = 20, 2, 1, 64, 700
+    M, KVH, hd, p0 = 20, 1, 64, 700
     _, q, kc, vc = _case(window % 1000 + path, M, H, KVH, hd, p0 + M, 1)
     pos, sl = p0 + np.arange(M), np.zeros(M)
     got = ec.attention_dev(q, kc, vc, pos, sl, H, KVH, window=window, path=path)
