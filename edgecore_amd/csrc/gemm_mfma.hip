@@ -630,25 +630,44 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
 
 template <int OP, int EPI>
 hipError_t launch_epi(const GemvArgs &a, int bm, hipStream_t s) {
-  // Row tiles by the number of blocks they give, K x N at M rows, us at 32 / 64
-  // / 128 rows.  int8 SwiGLU: 1536 x 8960 at 2048 140 / 92 / 85 (2240 blocks of
-  // 128), at 1024 61 / 45 / 45 (1120); 896 x 4864 at 777 21 / 18 / 23 (532),
-  // at 512 14 / 13 / 15, at 1500 30 at 128 (912) and 31 at 64; N = 896 at 2048 rows: 448 blocks of 32 beat 224 of 64
-  // (9.7 and 10.7, K = 4864 34.0 and 35.5).  The 16-bit parts double or triple
-  // the activation tile, so 128 rows leave one block per CU: fp16 896 x 4864
-  // SwiGLU at 777 44 / 40 / 64 (988 blocks of 64), at 512 30 / 33 / 45 (608),
-  // 1536 x 8960 at 2048 313 / 271 / 290, stores 1000 x 5000 at 640 38 / 32
-  // (400 of 64), GELU 768 x 3072 at 1024 36 / 40 (384); bf16 at 777 55 / 65 / 84, 1536 x 8960
-  // at 2048 410 / 446 / 383, 896 x 4864 at 2048 150 / 166 / 140 (1216 of 128);
-  // bf16 stores 896 x 9728 at 777 53 / 48 / 79, at 512 38 / 38 / 54.
+  // Row tiles by the blocks that 64 and 128 rows give.  The larger tile wins
+  // where its blocks fill the CUs' two slots (about 400 to 512 of them) or
+  // there are so many that the last round is a small part; in between its
+  // second round is mostly idle.  K x N at M rows, us at 32 / 64 / 128 rows (t64,
+  // t128 blocks), 142 shapes of each type and epilogue:
+  // int8: stores 1536 x 6466 at 967 24.4 / 23.8 / 19.7 (816, 408), 896 x 4864 at
+  // 777 12.2 / 10.7 / 13.3 (494, 266), 896 x 9728 at 2048 39 / 35 / 34 (2432,
+  // 1216), N = 896 at 2048 rows 9.7 / 10.7 (448 blocks of 32), K = 4864 34.0 /
+  // 35.5; SwiGLU 896 x 2048 at 2048 22 / 19.3 / 18.2 (1024, 512), 4864 x 1991 at
+  // 1572 70 / 56 / 44 (800, 416), 896 x 4864 at 777 21.7 / 19.3 / 26.2 (988, 532),
+  // 1536 x 8960 at 2048 140 / 92 / 85 (t128 2240); GELU as stores, but 128 rows
+  // no better at 400 to 512.
+  // The 16-bit parts double or triple the activation tile, so 128 rows leave
+  // one block per CU.  fp16: stores 1000 x 5000 at 640 37 / 26 / 32 (400, 200);
+  // GELU the same 51 / 44 / 55, 3840 x 2860 at 1276 111 / 87 / 100 (460, 230), 768
+  // x 3072 at 1024 35 / 39 / 47 (384, 192), 896 x 9728 at 512 50 / 56 / 86 (608,
+  // 304); SwiGLU 4864 x 896 at 2048 124 / 90 / 104 (448, 224), 896 x 1152 at 2048
+  // 35 / 39 / 51 (576, 288), 896 x 4864 at 777 45 / 41 / 65 (988, 532).  bf16:
+  // stores 896 x 1152 at 2048 35 / 30 / 34 (288, 144), 1536 x 2048 at 1024 29 / 33
+  // / 49 (256, 128); GELU 1000 x 5000 at 640 57 / 50 / 65 (400, 200), 896 x 9728
+  // at 512 59 / 63 / 101 (608, 304); SwiGLU 896 x 4864 at 777 57 / 65 / 84, 1536 x
+  // 8960 at 2048 410 / 446 / 383, 896 x 4864 at 2048 150 / 166 / 140 (t128 1216).
   constexpr int NOUT = EPI == EPI_SWIGLU ? kBN / 2 : kBN;
   const long gx = (a.N + NOUT - 1) / NOUT, t128 = gx * ((a.M + 127) / 128), t64 = gx * ((a.M + 63) / 64);
   if (bm == 0) {
-    constexpr bool heavy = EPI == EPI_SWIGLU || EPI == EPI_GELU;  // epilogues worth spreading
-    if (OP == OP_I8) bm = t128 >= 768 ? 128 : t64 >= 256 ? 64 : 32;
-    else if (OP == OP_F16) bm = t64 >= (heavy ? 800 : 256) ? 64 : 32;
-    else if (EPI == EPI_SWIGLU) bm = t128 >= 1200 ? 128 : 32;
-    else bm = t64 >= 500 ? 64 : 32;
+    // 64-row tiles: from `from` blocks to two per CU, and from `many` on
+    auto two_slots = [t64](int from, int many) { return (t64 >= from && t64 <= 512) || t64 >= many; };
+    constexpr bool store = EPI == EPI_STORE || EPI == EPI_RESID;
+    if (OP == OP_I8) {
+      if (t128 >= 768 || (EPI != EPI_GELU && t128 >= 400 && t128 <= 512)) bm = 128;
+      else bm = t64 >= 256 ? 64 : 32;
+    } else if (OP == OP_F16) {
+      bm = (store ? t64 >= 256 : EPI == EPI_GELU ? two_slots(400, 800) : two_slots(350, 640)) ? 64 : 32;
+    } else if (EPI == EPI_SWIGLU) {
+      bm = t128 >= 1200 ? 128 : 32;
+    } else {
+      bm = (store ? t64 > 256 : two_slots(390, 640)) ? 64 : 32;
+    }
   }
   if (bm == 128) return launch_bm<OP, 128, EPI>(a, s);
   if (bm == 64) return launch_bm<OP, 64, EPI>(a, s);

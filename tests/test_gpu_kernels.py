@@ -149,7 +149,7 @@ def test_dev_entry_points_reject_bad_shapes():
 # ec_gemm_int8_epi_dev runs the prefill linears' int8 matrix-core GEMM with
 # every fused epilogue and each row tile (32, 64, 128 rows), on shapes with
 # row and column tails; 0 lets the library pick, as the forward does (the
-# C4 shapes: gate/up of 2048 rows takes 128-row tiles, qkv 64-row tiles).
+# C4 shapes: gate/up of 2048 rows takes 128-row tiles, q|k|v 32-row tiles).
 TILE_SHAPES = [(200, 896, 300), (130, 1536, 129), (257, 64, 200), (64, 4864, 128)]
 
 
@@ -200,10 +200,14 @@ def test_gemm_int8_tiles_and_epilogues(bm, M, K, N):
     assert np.array_equal(_bits(swi), _bits(oracle.map_op(1, g) * u))
 
 
-@pytest.mark.parametrize("M,K,N", [(2048, 896, 2048), (1024, 1536, 4096), (1000, 896, 2120), (2040, 896, 2100)])
+@pytest.mark.parametrize("M,K,N", [(2048, 896, 2048), (1024, 1536, 4096), (1000, 896, 2120), (2040, 896, 2100),
+                                   (1000, 256, 6900), (2040, 128, 6200), (1000, 144, 6900), (1000, 128, 3300)])
 def test_gemm_int8_auto_tile_prefill_shapes(M, K, N):
-    """Shapes whose automatic tile is 128 rows (2048x2048, 1024x4096,
-    2040x2100) or 64 rows (1000x2120), with row and column tails."""
+    """Shapes with row and column tails whose automatic tile is, store and
+    SwiGLU, 64 and 128 rows (2048x2048, 1024x4096: 512 blocks of 128 rows for
+    SwiGLU), 64 (1000x2120, 2040x2100), 128 (1000x6900: 432 blocks for stores, 864
+    for SwiGLU, also with a row that ends inside a stage; 2040x6200: 784 and
+    1552) and 64 and 128 (1000x3300: 208 and 416)."""
     A, B, B2, a_s, b_s, b2_s, bias, C0 = _epi_inputs(M, K, N, seed=M ^ N)
     store = ec.gemm_int8_epi(0, 0, A, a_s, B, b_s, bias=bias)
     assert np.array_equal(_bits(store), _bits(oracle.gemm_int8(A, a_s, B, b_s, bias)))
@@ -289,6 +293,31 @@ def test_gemm_w16_tiles_and_epilogues(bm, M, K, N, bf16):
     want = _silu64(v) * u
     tol = 1.1 * (np.abs(u) * bv + np.abs(_silu64(v)) * bu) + 1e-6 * np.abs(want)
     check(ec.gemm_w16_epi(wt, 3, bm, A, B, B2=B2), want, tol)
+
+
+# row tiles that the library picks, by the blocks of 64 rows: stores 32 up to 255
+# (bf16 256) and 64 above; GELU 64 for 400 to 512 (bf16 390) and from 800 (640);
+# SwiGLU fp16 64 for 350 to 512 and from 640, bf16 32 and, from 1200 blocks of
+# 128 rows, 128.  Row and column tails, rows that end inside a stage.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1000, 64, 2040), (1020, 72, 2048), (630, 128, 5000), (510, 64, 9700),
+                                   (630, 64, 2300), (2040, 40, 4830)])
+def test_gemm_w16_auto_tiles(M, K, N, bf16):
+    wt = 2 if bf16 else 1
+    A, B, B2, bias, C0 = _w16_inputs(M, K, N, bf16, seed=M + K + N + bf16)
+    v, bv = _exact_and_bound(A, B, bf16)
+    b64, ulp = bias.astype(np.float64), 2.0 ** -23
+
+    def check(got, want, tol):
+        assert np.all(np.abs(got.astype(np.float64) - want) <= tol + 2 * ulp * np.abs(want) + 1e-30)
+
+    check(ec.gemm_w16_epi(wt, 4, 0, A, B, bias=bias), v + b64, bv)
+    check(ec.gemm_w16_epi(wt, 5, 0, A, B, bias=bias, C0=C0), C0.astype(np.float64) + (v + b64), bv)
+    check(ec.gemm_w16_epi(wt, 6, 0, A, B, bias=bias), _gelu64(v + b64), 1.2 * bv + 1e-6)
+    u, bu = _exact_and_bound(A, B2, bf16)
+    want = _silu64(v) * u
+    check(ec.gemm_w16_epi(wt, 3, 0, A, B, B2=B2), want,
+          1.1 * (np.abs(u) * bv + np.abs(_silu64(v)) * bu) + 1e-6 * np.abs(want))
 
 
 @pytest.mark.parametrize("bf16", [False, True])
