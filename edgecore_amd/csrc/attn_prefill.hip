@@ -16,7 +16,7 @@
 //
 // Two kernels: attn_prefill_mm_kernel (below), with the products on the matrix
 // cores, for spans of up to 4096 positions, and attn_prefill_kernel for longer
-// ones and for short prompts at head_dim 128.
+// ones and for prompts that are few blocks (mm_takes).
 //
 // attn_prefill_kernel: one block takes one query head and NW consecutive
 // tokens, one per wave (8, or 4 when the scores of 8 do not fit the LDS).  The
@@ -53,10 +53,10 @@ constexpr int kPfTile = 64;  // positions per staged K / V tile
 // time) both hit distinct banks.
 constexpr int pf_vrow(int d) { return d * (kPfTile + 4) + 4 * (d >> 3); }
 
-// NW waves per block, QW tokens per wave (consecutive), NW * QW tokens per block
-template <int HD, int NW, int QW>
+// NW waves per block, each with one token (consecutive)
+template <int HD, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int ngroups, int nsc) {
-  constexpr int NT = NW * 64, QB = NW * QW;
+  constexpr int NT = NW * 64;
   constexpr int KP = HD + 4;                   // floats per staged row
   constexpr int CPR = HD / 8;                  // 16-byte chunks (8 halves) per cache row
   constexpr int TCH = kPfTile * CPR;           // chunks per tile
@@ -72,46 +72,37 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int h = blockIdx.x;
   const int kvh = h * a.KVH / a.H;
-  const int m0 = (ngroups - 1 - (int)blockIdx.y) * QB;  // longest key ranges first
+  const int m0 = (ngroups - 1 - (int)blockIdx.y) * NW;  // longest key ranges first
   const int slot = ld_uniform(a.slot + m0);
-  const int pos_hi = ld_uniform(a.pos + min(m0 + QB - 1, a.M - 1));
+  const int pos_hi = ld_uniform(a.pos + min(m0 + NW - 1, a.M - 1));
   const int lo0 = a.window > 0 ? max(0, ld_uniform(a.pos + m0) - a.window + 1) : 0;
-  // this wave's tokens (tail waves repeat the last token and store nothing)
-  int pos[QW], lo[QW], mq[QW];
-  bool act[QW];
-  float *scq[QW];  // scores, then probabilities, of token i at index p - lo0
-#pragma unroll
-  for (int i = 0; i < QW; i++) {
-    const int m = m0 + QW * w + i;
-    act[i] = m < a.M;
-    mq[i] = min(m, a.M - 1);
-    pos[i] = ld_uniform(a.pos + mq[i]);
-    lo[i] = a.window > 0 ? max(0, pos[i] - a.window + 1) : 0;
-    scq[i] = lds + (kPfTile + 4) * KP + (QW * w + i) * nsc;
-  }
+  // this wave's token (tail waves repeat the last token and store nothing)
+  const bool act = m0 + w < a.M;
+  const int mq = min(m0 + w, a.M - 1);
+  const int pos = ld_uniform(a.pos + mq);
+  const int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  float *sc = lds + (kPfTile + 4) * KP + w * nsc;  // its scores, then probabilities, at index p - lo0
   if (t < 32) etab[t] = ec_exp2_32[t];
   const size_t cbase = (size_t)slot * a.C * a.kv + (size_t)kvh * HD;
   const uint16_t *Kc = a.kc + cbase, *Vc = a.vc + cbase;
 
   // q rows of the block's tokens through the (still free) tile area into
   // each wave's registers
-  for (int e = t; e < QB * HD / 4; e += NT) {
+  for (int e = t; e < NW * HD / 4; e += NT) {
     const int r = e / (HD / 4), c4 = e - r * (HD / 4);
     const float *qrow = a.q + (size_t)min(m0 + r, a.M - 1) * a.ldq + (size_t)h * HD;
     *reinterpret_cast<float4 *>(tile + r * HD + 4 * c4) = *reinterpret_cast<const float4 *>(qrow + 4 * c4);
   }
   __syncthreads();
-  float q[QW][HD];
+  float q[HD];
 #pragma unroll
-  for (int i = 0; i < QW; i++)
-#pragma unroll
-    for (int c4 = 0; c4 < HD / 4; c4++) {
-      const float4 v = *reinterpret_cast<const float4 *>(tile + (QW * w + i) * HD + 4 * c4);
-      q[i][4 * c4] = v.x;
-      q[i][4 * c4 + 1] = v.y;
-      q[i][4 * c4 + 2] = v.z;
-      q[i][4 * c4 + 3] = v.w;
-    }
+  for (int c4 = 0; c4 < HD / 4; c4++) {
+    const float4 v = *reinterpret_cast<const float4 *>(tile + w * HD + 4 * c4);
+    q[4 * c4] = v.x;
+    q[4 * c4 + 1] = v.y;
+    q[4 * c4 + 2] = v.z;
+    q[4 * c4 + 3] = v.w;
+  }
 
   // tile staging: the next tile's 16-byte chunks are loaded into registers
   // (gload) while the waves work on the current one, then converted to fp32
@@ -168,10 +159,8 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
     }
   };
 
-  // ---- scores: lane = position, the QW sequential dots share each K read ----
-  float mx[QW];
-#pragma unroll
-  for (int i = 0; i < QW; i++) mx[i] = -FLT_MAX;
+  // ---- scores: lane = position, one sequential dot each ----
+  float mx = -FLT_MAX;
   gload(Kc, lo0);
   for (int p0 = lo0; p0 <= pos_hi; p0 += kPfTile) {
     __syncthreads();  // the previous tile is consumed
@@ -181,46 +170,31 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
     if (p0 + kPfTile <= pos_hi) gload(Kc, p0 + kPfTile);
     else gload(Vc, lo0);
     const int p = p0 + lane;
-    if (p >= lo[0] && p <= pos[QW - 1]) {
+    if (p >= lo && p <= pos) {
       const float *kr = tile + lane * KP;
-      float s[QW];
-#pragma unroll
-      for (int i = 0; i < QW; i++) s[i] = 0.0f;
+      float s = 0.0f;
 #pragma unroll
       for (int c = 0; c < HD / 4; c++) {
         const float4 k4 = *reinterpret_cast<const float4 *>(kr + 4 * c);
         const float kk[4] = {k4.x, k4.y, k4.z, k4.w};
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-#pragma unroll
-          for (int i = 0; i < QW; i++) {
-            const float pr = q[i][4 * c + e] * kk[e];
-            s[i] = s[i] + pr;
-          }
+          const float pr = q[4 * c + e] * kk[e];
+          s = s + pr;
         }
       }
-      // every token's dot is formed in full, interleaved with the others;
-      // only the stores below depend on the token's range
-#pragma unroll
-      for (int i = 0; i < QW; i++) asm volatile("" : "+v"(s[i]));
-#pragma unroll
-      for (int i = 0; i < QW; i++) {
-        if (p >= lo[i] && p <= pos[i]) {
-          const float si = (float)((double)s[i] * a.inv_hd);
-          scq[i][p - lo0] = si;
-          mx[i] = fmaxf(mx[i], si);
-        }
-      }
+      const float si = (float)((double)s * a.inv_hd);
+      sc[p - lo0] = si;
+      mx = fmaxf(mx, si);
     }
   }
 
-  // ---- softmax of each of the wave's tokens ----
+  // ---- softmax of the wave's token ----
   __syncthreads();
-#pragma unroll
-  for (int i = 0; i < QW; i++) {
-    const float m = wave_max_dpp(mx[i]);
-    const int n = pos[i] - lo[i] + 1;
-    float *sq = scq[i] + (lo[i] - lo0);
+  {
+    const float m = wave_max_dpp(mx);
+    const int n = pos - lo + 1;
+    float *sq = sc + (lo - lo0);
     // four of the lane's scores per step, k, k + 64, k + 128, k + 192 (the
     // lane's order of its part of the sum); past n a score of -inf adds
     // exp = 0 (reads clamped to the token's last slot)
@@ -252,12 +226,10 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
     }
   }
 
-  // ---- output: lane = element d; per token, the sum over positions in order ----
-  float o[QW][DPL];
+  // ---- output: lane = element d, the sum over positions in order ----
+  float o[DPL];
 #pragma unroll
-  for (int i = 0; i < QW; i++)
-#pragma unroll
-    for (int j = 0; j < DPL; j++) o[i][j] = 0.0f;
+  for (int j = 0; j < DPL; j++) o[j] = 0.0f;
   const int d0 = HD >= 64 ? lane : (lane & (HD - 1));
   // this lane's element of the tile's position p at vt[p - p0] (of element
   // d0 + 64 j at vt[p - p0 + VJ * j])
@@ -267,40 +239,29 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
     lstore_v();
     __syncthreads();
     if (p0 + kPfTile <= pos_hi) gload(Vc, p0 + kPfTile);
-    // a position that only some tokens of the wave take
-    auto add_some = [&](int p) {
-      const float *vr = vt + (p - p0);
+    auto add1 = [&](int p) {
+      const float pr = sc[p - lo0], *vr = vt + (p - p0);
 #pragma unroll
-      for (int i = 0; i < QW; i++) {
-        if (p >= lo[i] && p <= pos[i]) {
-          const float pr = scq[i][p - lo0];
-#pragma unroll
-          for (int j = 0; j < DPL; j++) {
-            const float pv = pr * vr[VJ * j];
-            o[i][j] = o[i][j] + pv;
-          }
-        }
+      for (int j = 0; j < DPL; j++) {
+        const float pv = pr * vr[VJ * j];
+        o[j] = o[j] + pv;
       }
     };
-    const int r0 = max(p0, lo[0]), r1 = min(p0 + kPfTile - 1, pos[QW - 1]);
-    int c0 = max(p0, lo[QW - 1]), c1 = min(p0 + kPfTile - 1, pos[0]);  // taken by every token
-    if (c0 > c1) c0 = r1 + 1, c1 = r1;
+    const int r0 = max(p0, lo), r1 = min(p0 + kPfTile - 1, pos);
     int p = r0;
-    for (; p < c0; p++) add_some(p);
-    for (; p <= c1 && ((p - lo0) & 3); p++) add_some(p);
-    const int ng = p <= c1 ? (c1 - p + 1) >> 2 : 0;
+    for (; p <= r1 && ((p - lo0) & 3); p++) add1(p);
+    const int ng = p <= r1 ? (r1 - p + 1) >> 2 : 0;
     if (ng > 0) {
       // groups of 4 positions in two register sets (ping-pong): the
-      // probabilities (one 16-byte read per token) and V elements of the next
-      // group are read before the adds of the current one.  The look-ahead
-      // reads are unconditional; past c1 they reach at most 4 positions
-      // further: the tile's 4 spare rows, the next token's score slots or the
-      // 4 spare floats after the last token's (values not used).
-      float4 pa[QW], pb[QW];
+      // probabilities (one 16-byte read) and V elements of the next group are
+      // read before the adds of the current one.  The look-ahead reads are
+      // unconditional; past r1 they reach at most 4 positions further: the
+      // tile's 4 spare rows, the next token's score slots or the 4 spare floats
+      // after the last token's (values not used).
+      float4 pa, pb;
       float va[4][DPL], vb[4][DPL];
-      auto load4 = [&](int pp, float4 *pr, float (*vv)[DPL]) {
-#pragma unroll
-        for (int i = 0; i < QW; i++) pr[i] = *reinterpret_cast<const float4 *>(scq[i] + (pp - lo0));
+      auto load4 = [&](int pp, float4 &pr, float (*vv)[DPL]) {
+        pr = *reinterpret_cast<const float4 *>(sc + (pp - lo0));
         const float *vr = vt + (pp - p0);
 #pragma unroll
         for (int j = 0; j < DPL; j++) {
@@ -311,17 +272,14 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
           vv[3][j] = v4.w;
         }
       };
-      auto add4 = [&](const float4 *pr, float (*vv)[DPL]) {
+      auto add4 = [&](const float4 &pr, float (*vv)[DPL]) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
+          const float pe = e == 0 ? pr.x : e == 1 ? pr.y : e == 2 ? pr.z : pr.w;
 #pragma unroll
-          for (int i = 0; i < QW; i++) {
-            const float pe = e == 0 ? pr[i].x : e == 1 ? pr[i].y : e == 2 ? pr[i].z : pr[i].w;
-#pragma unroll
-            for (int j = 0; j < DPL; j++) {
-              const float pv = pe * vv[e][j];
-              o[i][j] = o[i][j] + pv;
-            }
+          for (int j = 0; j < DPL; j++) {
+            const float pv = pe * vv[e][j];
+            o[j] = o[j] + pv;
           }
         }
       };
@@ -341,15 +299,12 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
         if (++g == ng) break;
       }
     }
-    for (; p <= r1; p++) add_some(p);
+    for (; p <= r1; p++) add1(p);
   }
+  if (act && (HD >= 64 || lane < HD)) {
+    float *out = a.out + (size_t)mq * a.ldo + (size_t)h * HD + d0;
 #pragma unroll
-  for (int i = 0; i < QW; i++) {
-    if (act[i] && (HD >= 64 || lane < HD)) {
-      float *out = a.out + (size_t)mq[i] * a.ldo + (size_t)h * HD + d0;
-#pragma unroll
-      for (int j = 0; j < DPL; j++) out[64 * j] = o[i][j];
-    }
+    for (int j = 0; j < DPL; j++) out[64 * j] = o[j];
   }
 }
 
@@ -372,7 +327,11 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
 //   - scores: tile t of 64 positions belongs to wave t % 8, which keeps its
 //     16 x 64 scores in 16 registers per lane (up to NT tiles): scores never
 //     reach LDS, so two blocks share a CU where 16 tokens' scores of 2048
-//     positions (128 KB) left room for one.  B = the lane's position's k row,
+//     positions (128 KB) left room for one.  NT 1 and 2 (spans to 1024) hold
+//     them in registers; at NT 4, whose 64 are live beside 16 products twice
+//     and a tile's K or V in 128, the compiler spills 105 (232 bytes of scratch
+//     per lane; head_dim 128: 102 and 220), at NT 8 in 256 41 (104; 37 and 88).
+//     B = the lane's position's k row,
 //     A = four elements of the 16 tokens' q, one of them broadcast to the four
 //     blocks per product.  Register 4 b + r of lane l: token 4 (l / 16) + r,
 //     position 16 b + l % 16.
@@ -387,10 +346,11 @@ __global__ __launch_bounds__(NW * 64) void attn_prefill_kernel(AttnArgs a, int n
 // finite outside a token's range does not reach it.
 //
 // 2048 tokens, 14 heads of 64: 363 us with the scores in LDS and DPP products,
-// 251 (another card 266) here; 12 heads of 128: 667 and 317 us; 500 tokens, 14 heads: 55 and
-// 43 us.  The adds and products alone are about 125 us of that at 2.3 GHz, the
-// exponentials 25 us; the rest is the output phase's one wave per SIMD and
-// block (198 cycles per four positions where the SIMD could do 72).
+// 251 (another card 266) here; 12 heads of 128: 667 and 317 us; 500 tokens, 14
+// heads: 55 and 43 us.  The adds and products alone are about 125 us of that at
+// 2.3 GHz, the exponentials 25 us; the rest is the output phase's one wave per
+// SIMD and block (198 cycles per four positions where the SIMD could do 72) and
+// the spilled scores' way to scratch and back, which that count includes.
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -791,7 +751,7 @@ template <int HD, int NW>
 void launch_pf(const AttnArgs &a, hipStream_t st) {
   const int ngroups = (a.M + NW - 1) / NW;
   const dim3 grid(a.H, ngroups);
-  klaunch((attn_prefill_kernel<HD, NW, 1>), grid, dim3(NW * 64), pf_lds_bytes(a, NW) - 256, st, a, ngroups,
+  klaunch((attn_prefill_kernel<HD, NW>), grid, dim3(NW * 64), pf_lds_bytes(a, NW) - 256, st, a, ngroups,
           pf_nsc(a, NW));
 }
 
