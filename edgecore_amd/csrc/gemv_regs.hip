@@ -1,4 +1,4 @@
-// Linears with 16-bit weights and 3 to 15 fp32 activation rows (src/kernels.c:
+// Linears with 16-bit weights and 2 to 15 fp32 activation rows (src/kernels.c:
 // 129-151), above all the language-model head of batched decoding: the
 // activations in registers.
 //
@@ -172,13 +172,16 @@ bool gemv_regs_ok(const GemvArgs &a, int wt) {
          a.lda % 4 == 0 && !((uintptr_t)a.A & 15u) && !((uintptr_t)a.W & 15u) && !a.cand && !a.bias;
 }
 
-// From 4 rows on at every size, and from 2 for wide outputs.  Fused GEMV and
-// this kernel, us, K x N: 1536 x 4096 5.0 and 6.2 (2 rows), 5.8 and 6.3 (3),
-// 6.5 and 6.3 (4), 9.7 and 7.8 (8), 17.5 and 9.5 (15); 896 x 896 5.9 and 4.3
-// (4), 9.8 and 4.8 (8); 896 x 9728 6.6 and 5.9 (2), 13.7 and 8.1 (8); 896 x
-// 151936 62 and 47 (2), 99 and 48 (4), 153 and 64 (8), 282 and 124 (15).
+// From 4 rows on, and from 2 for wide outputs, of rows that give most lanes of a
+// wave a chunk (a row has 64 lanes here, in the fused GEMV as few as it needs).
+// Fused GEMV and this kernel, us, K x N: 1536 x 4096 5.0 and 6.2 (2 rows), 5.8
+// and 6.3 (3), 6.5 and 6.3 (4), 9.7 and 7.8 (8), 17.5 and 9.5 (15); 896 x 896
+// 5.9 and 4.3 (4), 9.8 and 4.8 (8); 896 x 9728 6.6 and 5.9 (2), 13.7 and 8.1 (8);
+// 896 x 151936 62 and 47 (2), 99 and 48 (4), 153 and 64 (8), 282 and 124 (15);
+// 128 x 20000 4.8 and 5.9 (2), 6.3 and 7.9 (5), 11.2 and 12.6 (12); 192 x 50257
+// 10.6 and 11.3 (2); 256 x 20000 5.2 and 5.9 (2).
 bool gemv_regs_faster(const GemvArgs &a, int wt) {
-  return gemv_regs_ok(a, wt) && (a.M >= 4 || (a.M >= 2 && a.N >= 8192));
+  return gemv_regs_ok(a, wt) && ((a.M >= 4 && a.K >= 192) || (a.M >= 2 && a.N >= 8192 && a.K >= 320));
 }
 
 hipError_t gemv_regs(const GemvArgs &a, int wt, hipStream_t s) {
