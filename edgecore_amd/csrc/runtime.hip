@@ -443,53 +443,45 @@ extern "C" int ec_gemm_int8_epi_dev(int epi, int bm, float *C, const int8_t *A, 
 
 // 16-bit parts of the kernel-ABI 16-bit GEMMs' activation rows, grown on demand.
 // A call captured on ec_stream() records a buffer's address in the caller's
-// graph, which may be replayed at any time: a buffer that a capture has seen is
-// not freed before ec_release.  A larger call retires it and takes twice its
-// size or more, so that all retired ones together are no larger than the one in
-// use (where the device has that much; else what the call needs).
+// graph, which may be replayed at any time, so a buffer is not freed before
+// ec_release: a larger call retires it and takes twice its size or more, so that
+// all retired ones together are no larger than the one in use (where the device
+// has that much; else what the call needs).
 struct W16Buf {
   void *p = nullptr;
-  size_t n = 0;           // bytes
-  bool recorded = false;  // a capture has seen p
+  size_t n = 0;  // bytes
   void *retired[64] = {};
   int nretired = 0;
 };
 static W16Buf g_w16_parts, g_w16_rs;
 
-static int w16_grow(W16Buf &b, size_t bytes, bool capturing) {
-  if (bytes > b.n) {
-    if (capturing)
-      return set_err(-3, "gemm: the workspace would grow inside a stream capture (run such a call before it)");
-    size_t want = bytes;
-    if (b.recorded) {
-      if (b.nretired == 64) return set_err(-3, "gemm: 64 workspaces are held for captured graphs");
-      b.retired[b.nretired++] = b.p;
-      want = bytes > 2 * b.n ? bytes : 2 * b.n;
-    } else if (b.p) {
-      EC_HIP(hipStreamSynchronize(g_stream));
-      EC_HIP(hipFree(b.p));
-    }
-    b.p = nullptr;
-    b.n = 0;
-    b.recorded = false;
-    if (want > bytes && dev_malloc(&b.p, want) != hipSuccess) {
-      (void)hipGetLastError();
-      b.p = nullptr;
-      want = bytes;
-    }
-    if (!b.p) EC_HIP(dev_malloc(&b.p, want));
-    b.n = want;
+static int w16_grow(W16Buf &b, size_t bytes) {
+  if (bytes <= b.n) return 0;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  EC_HIP(hipStreamIsCapturing(g_stream, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return set_err(-3, "gemm: the workspace would grow inside a stream capture (run such a call before it)");
+  size_t want = bytes;
+  if (b.p) {
+    if (b.nretired == 64) return set_err(-3, "gemm: 64 workspaces are held for captured graphs");
+    b.retired[b.nretired++] = b.p;
+    if (want < 2 * b.n) want = 2 * b.n;
   }
-  b.recorded = b.recorded || capturing;
+  b.p = nullptr;
+  b.n = 0;
+  if (want > bytes && dev_malloc(&b.p, want) != hipSuccess) {
+    (void)hipGetLastError();
+    b.p = nullptr;
+    want = bytes;
+  }
+  if (!b.p) EC_HIP(dev_malloc(&b.p, want));
+  b.n = want;
   return 0;
 }
 
 static int w16_workspace(int M, int ldp) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  EC_HIP(hipStreamIsCapturing(g_stream, &cap));
-  const bool capturing = cap != hipStreamCaptureStatusNone;
-  const int r = w16_grow(g_w16_parts, (size_t)M * 3 * ldp * sizeof(uint16_t), capturing);
-  return r ? r : w16_grow(g_w16_rs, (size_t)M * sizeof(float), capturing);
+  const int r = w16_grow(g_w16_parts, (size_t)M * 3 * ldp * sizeof(uint16_t));
+  return r ? r : w16_grow(g_w16_rs, (size_t)M * sizeof(float));
 }
 
 static int gemm_w16_dev(float *C, const float *A, const uint16_t *B, int M, int K, int N, bool bf16) {

@@ -123,8 +123,8 @@ void gemm_int8(float *C, const int8_t *A, const float *a_scale, const int8_t *B,
  * anything when a shape or pointer is invalid.  They may be captured on
  * ec_stream() and replayed there; those that use the library's workspace (the
  * 16-bit matrix-core kernel below) after a call of that size has run, since it
- * does not grow inside a capture.  A workspace that a capture has seen stays
- * until ec_release. */
+ * does not grow inside a capture.  A workspace that was outgrown stays until
+ * ec_release, for graphs that recorded it. */
 int ec_gemm_fp16_fp32_dev(float *C, const float *A, const uint16_t *B, int M, int K, int N);
 int ec_gemm_bf16_fp32_dev(float *C, const float *A, const uint16_t *B, int M, int K, int N);
 int ec_gemm_int8_dev(float *C, const int8_t *A, const float *a_scale, const int8_t *B,
