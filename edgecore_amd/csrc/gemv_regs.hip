@@ -178,10 +178,9 @@ bool gemv_regs_ok(const GemvArgs &a, int wt) {
 // and 6.3 (3), 6.5 and 6.3 (4), 9.7 and 7.8 (8), 17.5 and 9.5 (15); 896 x 896
 // 5.9 and 4.3 (4), 9.8 and 4.8 (8); 896 x 9728 6.6 and 5.9 (2), 13.7 and 8.1 (8);
 // 896 x 151936 62 and 47 (2), 99 and 48 (4), 153 and 64 (8), 282 and 124 (15);
-// 128 x 20000 4.8 and 5.9 (2), 6.3 and 7.9 (5), 11.2 and 12.6 (12); 192 x 50257
-// 10.6 and 11.3 (2); 256 x 20000 5.2 and 5.9 (2).
+// 128 x 20000 4.8 and 5.9 (2), 6.3 and 7.9 (5), 11.2 and 12.6 (12).
 bool gemv_regs_faster(const GemvArgs &a, int wt) {
-  return gemv_regs_ok(a, wt) && ((a.M >= 4 && a.K >= 192) || (a.M >= 2 && a.N >= 8192 && a.K >= 320));
+  return gemv_regs_ok(a, wt) && a.K >= 192 && (a.M >= 4 || (a.M >= 2 && a.N >= 8192));
 }
 
 hipError_t gemv_regs(const GemvArgs &a, int wt, hipStream_t s) {
