@@ -545,15 +545,25 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemvArgs a) {
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
-// K splits of a launch of T tiles over ns K stages: none when the tiles
-// already fill the CUs or the rows are short (under 16 stages: C2's q|k|v,
-// o and fc at 12 stages ran 8.6 -> 11.9, 8.6 -> 10.3 and 14.6 -> 18.7 us
-// split in 2-3); otherwise up to 256 blocks of 6 stages or more, within the
-// partial workspace, and no split left empty.  Only 32-row tiles split (few
-// tiles over long rows: a prefill of a few hundred tokens); such a launch
-// holds one block per CU and 4 stage buffers.
-int gemm_ksplit(int T, int ns, int BM) {
-  if (BM != 32 || T >= 128 || ns < 16 || T > kGmMaxTiles) return 1;
+// K splits of a launch of T tiles over ns K stages: none when the tiles already
+// fill the CUs or the rows are short (under 16 stages: C2's q|k|v, o and fc at 12
+// stages ran 8.6 -> 11.9, 8.6 -> 10.3 and 14.6 -> 18.7 us split in 2-3);
+// otherwise up to 256 blocks of 6 stages or more, within the partial workspace,
+// and no split left empty.  Only 32-row tiles split (few tiles over long rows: a
+// prefill of a few hundred tokens); such a launch holds one block per CU and 4
+// stage buffers.
+// Without a split such tiles are half as wide (launch_narrow).  For int8 that is
+// the faster form until a row's stages, run one after the other, take longer than
+// the split's meeting does, the later the fewer blocks a tile's stages are split
+// over (256 / T).  Split and not, us, at ns stages: 42 tiles (6 blocks) 12.6 and
+// 7.7 (16), 48 (5) 13.9 and 12.0 (38), 15.0 and 15.4 (52), 80 (3) 17.1 and 15.8
+// (52), 19.1 and 20.0 (70), 112 (2) 22.9 and 19.9 (70), 26.0 and 24.8 (90).
+// 16-bit weights would gain too (fp16 48 tiles of 24 stages 15.4 and 13.9), but
+// the split's shorter fp32 sums round less.
+int gemm_ksplit(int T, int ns, int BM, bool i8) {
+  if (BM != 32 || T >= 128 || T > kGmMaxTiles) return 1;
+  const int per = 256 / T;
+  if (ns < (!i8 ? 16 : per >= 5 ? 44 : per >= 3 ? 64 : 90)) return 1;
   int ks = min(min(ns / 6, 256 / T), 256 / BM);
   ks = min(ks, kGmPartInts / (T * BM * kBN));
   if (ks < 2) return 1;
@@ -565,8 +575,8 @@ int gemm_ksplit(int T, int ns, int BM) {
 // more than half of the CUs idle: twice the blocks, each with half the multiplies
 // and epilogue per stage.  128 x 768 x 3072 fp16 bias + GELU (96 tiles) 17.0 ->
 // 12.5 us, 100 x 896 x 896 bf16 (28) 13.2 -> 10.9, 100 x 1536 x 3000 int8 GELU
-// (96) 14.0 -> 9.4, 40 x 1536 x 4096 int8 (64) 8.1 -> 6.1.  Rows of 16 or more
-// stages split K first.
+// (96) 14.0 -> 9.4, 40 x 1536 x 4096 int8 (64) 8.1 -> 6.1.  Long rows split K
+// instead (gemm_ksplit).
 constexpr int kNarrowTiles = 128;
 
 template <int OP, int EPI>
@@ -591,7 +601,7 @@ hipError_t launch_bm(const GemvArgs &a, hipStream_t s) {
   // x 4856 x 896 bf16 67.9 us, 23.0 so; 120 x 8944 x 1536 int8 37.3 and 18.0.)
   const bool dl = (a.K * MfmaOp<OP>::EB) % 16 == 0 && (a.lda * MfmaOp<OP>::EB) % 16 == 0 && aligned16(a.A) &&
                   aligned16(a.W) && (EPI != EPI_SWIGLU || aligned16(a.W2));
-  const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM) : 1;
+  const int ks = dl ? gemm_ksplit(T, (a.K * MfmaOp<OP>::EB + kBK - 1) / kBK, BM, OP == OP_I8) : 1;
   const dim3 grid(8 * ((T + 7) / 8), ks);
   const bool part = (a.K * MfmaOp<OP>::EB) % kBK != 0;
   if constexpr (BM == 32) {

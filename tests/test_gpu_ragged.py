@@ -186,8 +186,9 @@ def test_w16_not_finite(M, bf16):
 
 # rows of whole 16-byte chunks that end inside a 128-byte stage of the tile
 # kernel: one chunk past and short of a stage, each row tile, split K (few
-# tiles, 16 or more stages), 2 to 4 stage buffers
-STAGE_SHAPES = [(33, 16, 40), (40, 112, 130), (40, 144, 130), (64, 2064, 200), (130, 4848, 129), (600, 1008, 9001)]
+# tiles, from 44 stages, 16-bit 16), 2 to 4 stage buffers
+STAGE_SHAPES = [(33, 16, 40), (40, 112, 130), (40, 144, 130), (64, 2064, 200), (130, 4848, 129), (64, 5520, 200),
+                (130, 6000, 129), (500, 11664, 896), (600, 1008, 9001)]
 
 
 @pytest.mark.parametrize("M,K,N", STAGE_SHAPES)
