@@ -37,6 +37,10 @@ MODEL_SPECS = {
                                ctx=128, vocab=1000, precision="int8"),
     "qwen2-ffn1040-int8": dict(arch="qwen2", layers=2, embd=256, heads=4, kv_heads=2, ffn=1040,
                                ctx=128, vocab=1000, precision="int8"),
+    # a vocabulary and width whose LM head keeps 5 to 15 rows in registers
+    "qwen2-head-int8": dict(arch="qwen2", layers=2, embd=256, heads=4, kv_heads=2, ffn=640, ctx=128, vocab=14001,
+                            precision="int8", tie=1),
+    "gpt2-head-fp16": dict(arch="gpt2", layers=2, embd=256, heads=4, ctx=128, vocab=14001, precision="fp16"),
     # long context: decode crosses 512-position boundaries
     "qwen2-long-int8": dict(arch="qwen2", layers=2, embd=128, heads=4, kv_heads=2, ffn=256,
                             ctx=1536, vocab=1000, precision="int8"),

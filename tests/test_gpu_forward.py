@@ -173,7 +173,13 @@ def test_graph_decode_equals_direct_and_oracle(make_model, name):
     assert np.array_equal(ids_graph, oids)
 
 
-@pytest.mark.parametrize("name,B", [("tiny-qwen2-int8", 3), ("tiny-gpt2-fp16", 16), ("qwen2-hd128-int8", 16)])
+# 5 to 15 tokens: int8 linears on the skinny matrix-core kernel with the fused
+# quantization, the LM head's rows in registers (qwen2-head, gpt2-head) and its
+# argmax over chunks
+@pytest.mark.parametrize("name,B", [("tiny-qwen2-int8", 3), ("tiny-gpt2-fp16", 16), ("qwen2-hd128-int8", 16),
+                                    ("tiny-gpt2-int8", 5), ("qwen2-head-int8", 5), ("qwen2-head-int8", 8),
+                                    ("qwen2-head-int8", 15), ("qwen2-hd128-int8", 9), ("gpt2-head-fp16", 6),
+                                    ("gpt2-head-fp16", 15)])
 def test_batched_graph_decode_equals_direct_and_oracle(make_model, name, B):
     """A greedy step of B tokens in B slots (argmax only) replays a HIP graph
     captured per (B, position bucket); asking for logits takes the direct

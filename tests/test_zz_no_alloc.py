@@ -1,7 +1,7 @@
 """ec_topk_dev_noalloc -- the device top-k selection with its scratch in the
 library's file-scope device array instead of allocations -- against
-ec_topk_dev, which allocates its scratch: identical values, indices and
-status, bit for bit, on two calls in a row, the second with a smaller input
+ec_topk_dev, which allocates its scratch and keeps it: identical values, indices
+and status, bit for bit, on two calls in a row, the second with a smaller input
 (fewer rows, a smaller vocabulary, a smaller k) than the first; a call
 needing more scratch than the array holds is refused with a message; and, as
 the first call into the library of a fresh process, on logits that the
