@@ -558,7 +558,7 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 // over (256 / T).  Split and not, us, at ns stages: 42 tiles (6 blocks) 12.6 and
 // 7.7 (16), 48 (5) 13.9 and 12.0 (38), 15.0 and 15.4 (52), 80 (3) 17.1 and 15.8
 // (52), 19.1 and 20.0 (70), 112 (2) 22.9 and 19.9 (70), 26.0 and 24.8 (90).
-// 16-bit weights would gain too (fp16 48 tiles of 24 stages 15.4 and 13.9), but
+// 16-bit weights would gain too (fp16 32 tiles of 24 stages 15.4 and 13.9), but
 // the split's shorter fp32 sums round less.
 int gemm_ksplit(int T, int ns, int BM, bool i8) {
   if (BM != 32 || T >= 128 || T > kGmMaxTiles) return 1;
